@@ -373,6 +373,41 @@ size_t oc_prefill_workspace_size(const oc_prefill_params* p);
 size_t oc_prefill_params_bytes(void);
 
 /*
+ * oc_prefill_gate -- the tile gate of the hook's prefill (perplexity_eval.py:
+ * 441-491) in two launches: q_norms = ||q[b, h, s]||_2 of every query row,
+ * k_norms = norm_scale * ||(W64 K_t)[48:64]||_F of every complete tile t <
+ * kv_len / 64, per (batch, kv head) qn = the max over its q heads of the
+ * lower median over positions of q_norms, and
+ *   mask[b, h, t] = qn * k_norms[b, h, t] <= tau_norm   (1 = evict; float64)
+ * with the statistics of oc_group_gate.  With cache given, the last batch
+ * element's k_norms also go to cache[h * cache_stride + t] and valid_tiles[h]
+ * (if given) is raised to the tile count.  What oc_band_norms, oc_row_norms,
+ * oc_kth_smallest and oc_group_gate do one by one.
+ */
+typedef struct oc_prefill_gate_params {
+  const void* q;                  /* (batch, num_q_heads, q_len, head_dim) */
+  int64_t q_stride_b, q_stride_h, q_stride_s;  /* elements; head_dim contiguous; rows 16-byte aligned */
+  const void* k;                  /* (batch, num_kv_heads, kv_len, head_dim) */
+  int64_t k_stride_b, k_stride_h, k_stride_s;
+  int32_t dtype;                  /* of q and k: OC_F32 / OC_F16 / OC_BF16 */
+  int32_t batch, num_q_heads, num_kv_heads, q_len, kv_len, head_dim;  /* head_dim 64 or 128 */
+  float norm_scale;
+  double tau_norm;                /* tau * 64 * head_dim */
+  float* q_norms;                 /* (batch, num_q_heads, q_len) */
+  float* k_norms;                 /* (batch, num_kv_heads, kv_len / 64) */
+  uint8_t* mask;                  /* (batch, num_kv_heads, kv_len / 64) */
+  float* gate_stats;              /* (batch, num_kv_heads, 3) or NULL */
+  float* cache;                   /* norm cache rows of the kv heads, or NULL */
+  int64_t cache_stride;           /* elements, >= kv_len / 64 */
+  int32_t* valid_tiles;           /* (num_kv_heads) or NULL */
+} oc_prefill_gate_params;
+
+int oc_prefill_gate(const oc_prefill_gate_params* p, void* stream);
+
+/* sizeof(oc_prefill_gate_params) as compiled, for binding checks */
+size_t oc_prefill_gate_params_bytes(void);
+
+/*
  * oc_block_spectra -- statistics of the normalised natural-order 512-point
  * Walsh-Hadamard transform X = H512 K_b / sqrt(512) of every 512-token
  * block b and head h of K (seq, num_heads, head_dim), as written by

@@ -3275,26 +3275,19 @@ __global__ __launch_bounds__(kThreads) void fwht_kernel(const DecodeArgs a) {
   }
 }
 
-// Band norms ||(W64 K_t)[band_lo, band_hi)||_F of tiles [t0, t0 + tcnt) of
-// every row (norm_cache.py:58-117), float32, clamped to 0 below 1e-38 as
-// the reference does; the full 64-point transform in registers as in
-// fwht_kernel, then the squares of the band's rows.  Tiles not wholly
-// inside the row's length are not written.
+// ||(W64 K_t)[lo, hi)||_F of one tile by one wave (in every lane), float32,
+// clamped to 0 below 1e-38 as the reference does (norm_cache.py:58-117): the
+// full 64-point transform in registers as in fwht_kernel, then the squares
+// of the band's rows.
 template <int DT, int D, bool PAGED>
-__global__ __launch_bounds__(kThreads) void band_norm_kernel(const DecodeArgs a) {
+__device__ __forceinline__ float band_norm_tile(const DecodeArgs& a, const RowInfo& ri, int row, int t, int band_lo,
+                                                int band_hi, const Deq& dq, int lane) {
   constexpr int CPL = D / 16;
   using L = Lay<DT, D>;
-  const int lane = threadIdx.x & 63;
-  const int64_t job = (int64_t)blockIdx.x * kWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (job >= (int64_t)a.num_rows * a.tcnt) return;
-  const int row = (int)(job / a.tcnt);
-  const int t = a.t0 + (int)(job - (int64_t)row * a.tcnt);
-  const RowInfo ri = row_info(a, row);
-  if ((t + 1) * 64 > ri.n_tok) return;
   uint32_t kw[16][L::LW];
   float f[16][CPL];
   load_tile<DT, D, PAGED>(a, ri, row, t, false, lane, kw);
-  decode_tile<DT, D>(kw, f, tile_kdeq(a, row, t));
+  decode_tile<DT, D>(kw, f, dq);
 #pragma unroll
   for (int h = 1; h < 16; h <<= 1) {
 #pragma unroll
@@ -3313,7 +3306,7 @@ __global__ __launch_bounds__(kThreads) void band_norm_kernel(const DecodeArgs a)
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
-    const bool in = 4 * i + gamma >= a.band_lo && 4 * i + gamma < a.band_hi;
+    const bool in = 4 * i + gamma >= band_lo && 4 * i + gamma < band_hi;
 #pragma unroll
     for (int c = 0; c < CPL; ++c) {
       float x = butterfly_rows<16>(f[i][c]);
@@ -3321,8 +3314,23 @@ __global__ __launch_bounds__(kThreads) void band_norm_kernel(const DecodeArgs a)
       ss = in ? __builtin_fmaf(x, x, ss) : ss;
     }
   }
-  float n = __builtin_sqrtf(wave_sum(ss));
-  if ((double)n < 1e-38) n = 0.f;
+  const float n = __builtin_sqrtf(wave_sum(ss));
+  return (double)n < 1e-38 ? 0.f : n;
+}
+
+// Band norms of tiles [t0, t0 + tcnt) of every row.  Tiles not wholly inside
+// the row's length are not written.
+template <int DT, int D, bool PAGED>
+__global__ __launch_bounds__(kThreads) void band_norm_kernel(const DecodeArgs a) {
+  const int lane = threadIdx.x & 63;
+  const int64_t job = (int64_t)blockIdx.x * kWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (job >= (int64_t)a.num_rows * a.tcnt) return;
+  const int row = (int)(job / a.tcnt);
+  const int t = a.t0 + (int)(job - (int64_t)row * a.tcnt);
+  const RowInfo ri = row_info(a, row);
+  if ((t + 1) * 64 > ri.n_tok) return;
+  const float n =
+      band_norm_tile<DT, D, PAGED>(a, ri, row, t, a.band_lo, a.band_hi, tile_kdeq(a, row, t), lane);
   if (lane == 0) {
     a.o_norm[(int64_t)row * a.o_stride + t] = n;
     if (a.o_valid) atomicMax(a.o_valid + row, t + 1);

@@ -714,45 +714,198 @@ __global__ __launch_bounds__(256) void row_norms_kernel(const char* x, int dtype
   if (lane == 0) out[r] = n;
 }
 
-// k-th smallest (0-based) of n non-negative floats per row by a radix
-// select over their bit patterns (monotone for x >= 0; NaN sorts last):
-// four 8-bit passes, each a 256-bin LDS histogram, then the bin holding
-// rank k.  One workgroup per row.
-__global__ __launch_bounds__(256) void kth_smallest_kernel(const float* x, int64_t n, int64_t row_stride, int64_t k,
-                                                           float* out) {
-  __shared__ uint32_t hist[256];
-  __shared__ uint32_t sel[2];
-  const float* row = x + (int64_t)blockIdx.x * row_stride;
-  uint32_t prefix = 0, pmask = 0;
-  uint64_t rank = (uint64_t)k;
-  for (int shift = 24; shift >= 0; shift -= 8) {
-    hist[threadIdx.x] = 0;
+// Exact selection by rank.  A workgroup of kSelWaves waves finds the k-th
+// smallest (0-based) of each of up to kSelRows rows of n non-negative floats
+// at once, an equal share of the waves per row, by a radix select over the
+// bit patterns (monotone for x >= 0; NaN sorts last).
+//
+// The values are norms of like vectors, so they share their leading bits: a
+// radix from bit 31 down puts every value into the same few bins, and the
+// LDS atomics of a pass then run one after another (the four 8-bit passes
+// with a one-thread bin scan took 35 us for 32 rows of 4096 norms).  Here
+// the digits are of u - min u, over the bits that max u - min u has, so one
+// pass of 1024 bins leaves a handful of values; once they are at most 64, one
+// wave ranks them directly, and only rows of many equal or clustered values
+// take further passes.  Values are read once and kept in registers (up to
+// 16 a lane; longer rows are read again in each pass).
+constexpr int kSelWaves = 16;
+constexpr int kSelThreads = kSelWaves * kWave;
+constexpr int kSelRows = 8;
+constexpr int kSelBits = 10;
+constexpr int kSelHeld = 16;
+
+struct SelLds {
+  __attribute__((aligned(16))) uint32_t hist[kSelRows][1 << kSelBits];
+  uint32_t cand[kSelRows][kWave];       // the values that share the digits found
+  uint32_t ncand[kSelRows];
+  uint32_t lo[kSelRows], hi[kSelRows];  // smallest and largest bit pattern of the row
+  uint32_t bin[kSelRows], cnt[kSelRows];  // the pass's digit and its values, and the values of the row below them
+  uint64_t below[kSelRows];
+  int open;  // rows not yet found
+};
+
+// largest x of the wave in lane 63 (the lanes of wave_incl_scan)
+__device__ __forceinline__ uint32_t wave_umax63(uint32_t x) {
+  auto step = [&](uint32_t y) { x = max(x, y); };
+  step((uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, 0x111, 0xF, 0xF, false));
+  step((uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, 0x112, 0xF, 0xF, false));
+  step((uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, 0x114, 0xF, 0xF, false));
+  step((uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, 0x118, 0xF, 0xF, false));
+  step((uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, 0x142, 0xA, 0xF, false));
+  step((uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, 0x143, 0xC, 0xF, false));
+  return x;
+}
+
+// out[r] (LDS, rows entries) = the k-th smallest of x[r * stride .. + n);
+// every thread of the workgroup calls it, rows <= kSelRows, k < n; out is
+// readable by all on return
+__device__ __forceinline__ void select_rows(const float* x, int64_t stride, int rows, int64_t n, uint64_t k, SelLds& s,
+                                            float* out) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wl = rows > 4 ? 1 : (rows > 2 ? 2 : (rows > 1 ? 3 : 4));  // log2 of the waves per row
+  const int r = (tid >> 6) >> wl;
+  const int64_t t0 = tid & ((kWave << wl) - 1), step = kWave << wl;
+  const bool first = t0 < kWave;  // the row's first wave
+  bool on = r < rows;             // the row has waves here and is not found yet
+  const float* xr = x + (on ? (int64_t)r * stride : 0);
+  const bool held = n <= kSelHeld * step;
+  uint32_t v[kSelHeld];
+  if (held) {
+#pragma unroll
+    for (int i = 0; i < kSelHeld; ++i) v[i] = __float_as_uint(xr[min(t0 + i * step, n - 1)]);
+  }
+  auto each = [&](auto f) {
+    if (held) {
+#pragma unroll
+      for (int i = 0; i < kSelHeld; ++i)
+        if (t0 + i * step < n) f(v[i]);
+    } else {
+      for (int64_t j = t0; j < n; j += step) f(__float_as_uint(xr[j]));
+    }
+  };
+  if (tid < kSelRows) {
+    s.lo[tid] = ~0u;
+    s.hi[tid] = 0u;
+    if (tid == 0) s.open = rows;
+  }
+  __syncthreads();
+  if (on) {
+    uint32_t mn = ~0u, mx = 0u;
+    each([&](uint32_t u) {
+      mn = min(mn, u);
+      mx = max(mx, u);
+    });
+    mn = ~wave_umax63(~mn);
+    mx = wave_umax63(mx);
+    if (lane == 63) {
+      atomicMin(&s.lo[r], mn);
+      atomicMax(&s.hi[r], mx);
+    }
+  }
+  __syncthreads();
+  const uint32_t lo = on ? s.lo[r] : 0u;
+  const uint32_t range = on ? s.hi[r] - lo : 0u;
+  int rb = range ? 32 - __builtin_clz(range) : 0;  // bits of the row's value still open
+  uint32_t prefix = 0;                             // the bits found, in place
+  uint64_t rank = k;                               // among the values that share them
+  while (true) {
+    const int sh = max(rb - kSelBits, 0);
+    for (int i = tid; i < rows << kSelBits; i += kSelThreads) (&s.hist[0][0])[i] = 0u;
+    if (tid < kSelRows) s.ncand[tid] = 0u;
     __syncthreads();
-    for (int64_t j = threadIdx.x; j < n; j += 256) {
-      const uint32_t u = __float_as_uint(row[j]);
-      if ((u & pmask) == prefix) atomicAdd(&hist[(u >> shift) & 255u], 1u);
+    // (d ^ prefix) >> rb == 0: d has the digits found (64 bits: rb may be 32)
+    auto shares = [&](uint32_t d) { return ((uint64_t)(d ^ prefix) >> rb) == 0; };
+    if (on) {
+      const uint32_t mask = (1u << (rb - sh)) - 1u;
+      each([&](uint32_t u) {
+        const uint32_t d = u - lo;
+        if (shares(d)) atomicAdd(&s.hist[r][(d >> sh) & mask], 1u);
+      });
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-      uint64_t acc = 0;
-      int bin = 255;
-      for (int i = 0; i < 256; ++i) {
-        if (acc + hist[i] > rank) {
-          bin = i;
-          break;
-        }
-        acc += hist[i];
+    if (on && first) {
+      // lane i holds bins 16 i .. 16 i + 15
+      constexpr int BPL = (1 << kSelBits) / kWave;
+      uint32_t c[BPL];
+      uint64_t sum = 0;
+#pragma unroll
+      for (int i = 0; i < BPL; i += 4) {
+        const uint4 w = *reinterpret_cast<const uint4*>(&s.hist[r][lane * BPL + i]);
+        c[i] = w.x, c[i + 1] = w.y, c[i + 2] = w.z, c[i + 3] = w.w;
+        sum += (uint64_t)w.x + w.y + w.z + w.w;
       }
-      sel[0] = (uint32_t)bin;
-      sel[1] = (uint32_t)(rank - acc);
+      uint64_t incl = sum;
+      if (n <= 0x7FFFFFFF) {
+        incl = (uint32_t)wave_incl_scan((int)sum);
+      } else {
+        for (int o = 1; o < 64; o <<= 1) {
+          const uint64_t up = __shfl_up((unsigned long long)incl, o, 64);
+          if (lane >= o) incl += up;
+        }
+      }
+      uint64_t acc = incl - sum;
+      if (acc <= rank && rank < incl) {  // one lane: the bins hold every value that shares the prefix
+        uint32_t bin = 0, cnt = 0;
+        uint64_t below = acc;
+#pragma unroll
+        for (int i = 0; i < BPL; ++i) {
+          if (acc <= rank) {
+            bin = lane * BPL + i;
+            below = acc;
+            cnt = c[i];
+          }
+          acc += c[i];
+        }
+        s.bin[r] = bin;
+        s.cnt[r] = cnt;
+        s.below[r] = below;
+      }
     }
     __syncthreads();
-    prefix |= sel[0] << shift;
-    pmask |= 255u << shift;
-    rank = sel[1];
+    bool few = false;
+    if (on) {
+      prefix |= s.bin[r] << sh;
+      rank -= s.below[r];
+      rb = sh;
+      few = rb > 0 && s.cnt[r] <= kWave;
+      if (few)
+        each([&](uint32_t u) {
+          if (shares(u - lo)) s.cand[r][atomicAdd(&s.ncand[r], 1u)] = u;
+        });
+    }
+    __syncthreads();
+    if (on && (few || rb == 0)) {
+      if (first) {
+        if (few) {
+          const int c = (int)s.cnt[r];
+          const uint32_t mine = s.cand[r][lane];
+          uint32_t under = 0;
+          for (int j = 0; j < c; ++j) {
+            const uint32_t o = s.cand[r][j];
+            under += (o < mine || (o == mine && j < lane)) ? 1u : 0u;
+          }
+          if (lane < c && under == (uint32_t)rank) out[r] = __uint_as_float(mine);
+        } else if (lane == 0) {
+          out[r] = __uint_as_float(lo + prefix);
+        }
+        if (lane == 0) atomicSub(&s.open, 1);
+      }
+      on = false;
+    }
+    __syncthreads();
+    // every pass takes bits off each row that is left, so all are found in at most four
+    if (s.open == 0) break;
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[blockIdx.x] = __uint_as_float(prefix);
+}
+
+// One workgroup per row (select_rows).
+__global__ __launch_bounds__(kSelThreads) void kth_smallest_kernel(const float* x, int64_t n, int64_t row_stride,
+                                                                   int64_t k, float* out) {
+  __shared__ SelLds s;
+  __shared__ float sel;
+  select_rows(x + (int64_t)blockIdx.x * row_stride, 0, 1, n, (uint64_t)k, s, &sel);
+  if (threadIdx.x == 0) out[blockIdx.x] = sel;
 }
 
 // The group norm of G per-head norms: their max (NaN-propagating) or the
@@ -777,16 +930,18 @@ __device__ float group_norm(const float* qh, int G, int reduce) {
   return qn;
 }
 
-// The tile gate of one (batch, kv head) by a 256-thread workgroup:
+// The tile gate of one (batch, kv head) by a workgroup of NT threads:
 // mask[t] = qn * kn[t] <= tau_norm for t < num_tiles and 0 up to mask_cols
 // (keep_pol: 1 = attend instead); with stats, the evicted count, qn and the
 // largest kn of the complete tiles (NaN if any is NaN, -inf if none).
+template <int NT>
 __device__ void gate_tiles(float qn, const float* knr, int num_tiles, int mask_cols, double tau_norm, int keep_pol,
                            uint8_t* mr, float* stats) {
-  __shared__ float s_red[2][4];
+  constexpr int NW = NT / kWave;
+  __shared__ float s_red[2][NW];
   float nev = 0.f, kmax = -__builtin_inff();
   bool knan = false;
-  for (int t = threadIdx.x; t < mask_cols; t += 256) {
+  for (int t = threadIdx.x; t < mask_cols; t += NT) {
     const bool full = t < num_tiles;
     // the reference compares (qn * kn) / (64 d) <= tau in float64 with
     // float32 norms; 64 d is a power of two, so that is qn * kn <= tau * 64 d
@@ -804,18 +959,22 @@ __device__ void gate_tiles(float qn, const float* knr, int num_tiles, int mask_c
     nev = wave_sum(nev);
     kmax = wave_max(kmax);
     const bool wnan = __ballot(knan) != 0;
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    if (lane == 0) {
       s_red[0][w] = nev;
       s_red[1][w] = wnan ? __builtin_nanf("") : kmax;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-      stats[0] = s_red[0][0] + s_red[0][1] + s_red[0][2] + s_red[0][3];
-      stats[1] = qn;
-      float m = s_red[1][0];
-      for (int i = 1; i < 4; ++i) m = (__builtin_isnan(m) || __builtin_isnan(s_red[1][i])) ? __builtin_nanf("") : fmaxf(m, s_red[1][i]);
-      stats[2] = m;
+    if (w == 0) {
+      const float wm = lane < NW ? s_red[1][lane] : -__builtin_inff();
+      const float n = wave_sum(lane < NW ? s_red[0][lane] : 0.f);
+      const bool nan = __ballot(__builtin_isnan(wm)) != 0;
+      const float m = wave_max(wm);
+      if (lane == 0) {
+        stats[0] = n;
+        stats[1] = qn;
+        stats[2] = nan ? __builtin_nanf("") : m;
+      }
     }
   }
 }
@@ -837,7 +996,7 @@ __global__ __launch_bounds__(256) void group_gate_kernel(const float* qn_heads, 
     if (qn_out) qn_out[bk] = qn;
   }
   __syncthreads();
-  gate_tiles(s_qn, kn + (int64_t)b * kn_sb + (int64_t)kv * kn_sh, num_tiles, mask_cols, tau_norm, keep_pol,
+  gate_tiles<256>(s_qn, kn + (int64_t)b * kn_sb + (int64_t)kv * kn_sh, num_tiles, mask_cols, tau_norm, keep_pol,
              mask + (int64_t)b * m_sb + (int64_t)kv * m_sh, stats ? stats + (int64_t)bk * 3 : nullptr);
 }
 
@@ -863,8 +1022,126 @@ __global__ __launch_bounds__(256) void hook_gate_kernel(const char* q, int dtype
   __syncthreads();
   if (threadIdx.x == 0) s_qn = group_norm(s_qh, G, OC_GROUP_MEDIAN);
   __syncthreads();
-  gate_tiles(s_qn, kn + (int64_t)kv * kn_sh, num_tiles, mask_cols, tau_norm, 1, mask + (int64_t)bk * m_sh,
+  gate_tiles<256>(s_qn, kn + (int64_t)kv * kn_sh, num_tiles, mask_cols, tau_norm, 1, mask + (int64_t)bk * m_sh,
              stats ? stats + (int64_t)bk * 3 : nullptr);
+}
+
+// ------------------------------------------------ the hook's prefill gate
+//
+// Two launches give everything that the prefill's tile gate needs: the norms
+// of q's rows and of K's tiles (one pass over each), then per (batch, kv
+// head) the medians, the gate, the statistics and the norm cache.
+
+struct PfGateArgs {
+  const char* q;
+  const char* k;
+  int64_t q_sb, q_sh, q_ss;  // byte strides (batch, head, position)
+  int64_t k_sb, k_sh, k_ss;
+  int32_t B, Hq, Hkv, G, Sq, T;
+  int32_t kblocks;  // workgroups of prefill_norms_kernel on K's tiles; the rest take q
+  int32_t qchunks;  // q workgroups per (batch, head)
+  float norm_scale;
+  double tau_norm;
+  float* qn;  // (B, Hq, Sq)
+  float* kn;  // (B, Hkv, T)
+  uint8_t* mask;
+  float* stats;
+  float* cache;  // kv head h's norms of the last batch element at cache[h * cache_stride], if given
+  int64_t cache_stride;
+  int32_t* valid;
+};
+
+// q's rows per workgroup of prefill_norms_kernel: a wave holds 64 / LPR rows
+// per 16-byte load of its lanes, kPnLoads loads in flight.
+constexpr int kPnLoads = 8;
+template <int DT, int D>
+constexpr int kPnLpr = D * (DT == OC_F32 ? 4 : 2) / 16;  // lanes per row
+template <int DT, int D>
+constexpr int kPnRows = kWaves * (kWave / kPnLpr<DT, D>) * kPnLoads;
+
+// ||q_s||_2 of every query row and norm_scale ||(W64 K_t)[48, 64)||_F of every
+// complete K tile.  Bound by the bytes of q (and of K, where the heads are
+// not grouped), so q is read in 16-byte pieces, several rows a load.  For 32
+// heads x 4096 rows of 256 bytes (33.5 MB) and 8 heads of K (8.4 MB) it takes
+// 9.6 us (4.4 TB/s); row_norms_kernel, one wave per row and two bytes a lane,
+// took 34 us for q alone, and band_norm_kernel 8.7 us for K.
+template <int DT, int D>
+__global__ __launch_bounds__(kThreads) void prefill_norms_kernel(const PfGateArgs a) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if ((int)blockIdx.x < a.kblocks) {
+    const int64_t job = (int64_t)blockIdx.x * kWaves + wave;
+    if (job >= (int64_t)a.B * a.Hkv * a.T) return;
+    const int row = (int)(job / a.T);
+    const int t = (int)(job - (int64_t)row * a.T);
+    DecodeArgs ka;  // what load_tile reads of contiguous rows
+    ka.k = a.k + (int64_t)(row / a.Hkv) * a.k_sb + (int64_t)(row % a.Hkv) * a.k_sh;
+    ka.k_row_stride = 0;
+    ka.k_tok_stride = a.k_ss;
+    const float n = band_norm_tile<DT, D, false>(ka, RowInfo{a.T * 64, a.T, 0, 0}, 0, t, 48, 64, Deq{1.f, false}, lane);
+    if (lane == 0) a.kn[job] = n * a.norm_scale;
+    return;
+  }
+  constexpr int LPR = kPnLpr<DT, D>;
+  constexpr int EPL = DT == OC_F32 ? 4 : 8;  // elements per lane
+  const int blk = blockIdx.x - a.kblocks;
+  const int bh = blk / a.qchunks;
+  const int s0 = (blk - bh * a.qchunks) * kPnRows<DT, D> + wave * (kPnRows<DT, D> / kWaves) + lane / LPR;
+  const char* base = a.q + (int64_t)(bh / a.Hq) * a.q_sb + (int64_t)(bh % a.Hq) * a.q_sh + 16 * (lane % LPR);
+  uint4 w[kPnLoads];
+#pragma unroll
+  for (int u = 0; u < kPnLoads; ++u)
+    w[u] = *reinterpret_cast<const uint4*>(base + (int64_t)min(s0 + u * (kWave / LPR), a.Sq - 1) * a.q_ss);
+#pragma unroll
+  for (int u = 0; u < kPnLoads; ++u) {
+    const uint32_t ww[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) {
+      const float x = elem<DT>(ww, e);
+      ss = __builtin_fmaf(x, x, ss);
+    }
+    if constexpr (LPR >= 16) ss += xpair<8>(ss);
+    ss += xpair<4>(ss);
+    ss += xpair<2>(ss);
+    ss += xpair<1>(ss);
+    if constexpr (LPR >= 32) ss += xpair<16>(ss);
+    const int s = s0 + u * (kWave / LPR);
+    if (lane % LPR == 0 && s < a.Sq) a.qn[(int64_t)bh * a.Sq + s] = __builtin_sqrtf(ss);
+  }
+}
+
+// Per (batch, kv head): the lower median over positions of each of its G q
+// heads' norms, their max (NaN propagates), the tile gate and its
+// statistics; the last batch element's tile norms go to the norm cache (as
+// the reference's loop over the batch leaves them, perplexity_eval.py:472-477).
+// A few workgroups, each a chain of short steps (11.5 us for 8 kv heads of 4
+// x 4096 norms): a select over 32 workgroups (35 us), the gate (4 us) and ten
+// small torch kernels for the scale, the cache and the statistics before.
+__global__ __launch_bounds__(kSelThreads) void prefill_gate_kernel(const PfGateArgs a) {
+  __shared__ SelLds s;
+  __shared__ float med[kSelRows];
+  const int bk = blockIdx.x;
+  const int b = bk / a.Hkv, kv = bk % a.Hkv;
+  bool nan = false;
+  float qn = -__builtin_inff();
+  for (int g0 = 0; g0 < a.G; g0 += kSelRows) {
+    const int rows = min(kSelRows, a.G - g0);
+    select_rows(a.qn + ((int64_t)b * a.Hq + (int64_t)kv * a.G + g0) * a.Sq, a.Sq, rows, a.Sq,
+                (uint64_t)(a.Sq - 1) / 2, s, med);
+    for (int g = 0; g < rows; ++g) {
+      nan = nan || __builtin_isnan(med[g]);
+      qn = med[g] > qn ? med[g] : qn;
+    }
+    __syncthreads();  // med is read before the next heads' are written
+  }
+  if (nan) qn = __builtin_nanf("");
+  const float* knr = a.kn + (int64_t)bk * a.T;
+  gate_tiles<kSelThreads>(qn, knr, a.T, a.T, a.tau_norm, 0, a.mask + (int64_t)bk * a.T, a.stats ? a.stats + 3 * bk : nullptr);
+  if (a.cache && b == a.B - 1) {
+    for (int t = threadIdx.x; t < a.T; t += kSelThreads) a.cache[(int64_t)kv * a.cache_stride + t] = knr[t];
+    if (threadIdx.x == 0 && a.valid) a.valid[kv] = max(a.valid[kv], a.T);
+  }
 }
 
 bool pf_float_dtype(int dt) { return dt == OC_F32 || dt == OC_F16 || dt == OC_BF16; }
@@ -881,6 +1158,14 @@ int launch_prefill(const PrefillArgs& a, hipStream_t s, unsigned blocks) {
   }
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? OC_OK : hip_fail(e, "prefill launch");
+}
+
+template <int DT, int D>
+void launch_prefill_norms(PfGateArgs& a, hipStream_t s) {
+  a.kblocks = (int)(((int64_t)a.B * a.Hkv * a.T + kWaves - 1) / kWaves);
+  a.qchunks = (a.Sq + kPnRows<DT, D> - 1) / kPnRows<DT, D>;
+  const unsigned blocks = (unsigned)(a.kblocks + (int64_t)a.B * a.Hq * a.qchunks);
+  hipLaunchKernelGGL((prefill_norms_kernel<DT, D>), dim3(blocks), dim3(kThreads), 0, s, a);
 }
 
 template <int DT>
@@ -1089,7 +1374,7 @@ extern "C" int oc_kth_smallest(const float* x, int64_t rows, int64_t n, int64_t 
   if (rows < 0 || n < 1 || k < 0 || k >= n || row_stride < n) return fail(OC_ERR_INVALID, "bad sizes (k must be < n)");
   if (rows > 0x7FFFFFFF) return fail(OC_ERR_UNSUPPORTED, "too many rows");
   if (rows == 0) return OC_OK;
-  hipLaunchKernelGGL(kth_smallest_kernel, dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream, x, n, row_stride,
+  hipLaunchKernelGGL(kth_smallest_kernel, dim3((unsigned)rows), dim3(kSelThreads), 0, (hipStream_t)stream, x, n, row_stride,
                      k, out);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? OC_OK : hip_fail(e, "select launch");
@@ -1113,6 +1398,54 @@ extern "C" int oc_group_gate(const float* q_norms, int32_t batch, int32_t num_kv
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? OC_OK : hip_fail(e, "group-gate launch");
 }
+
+extern "C" int oc_prefill_gate(const oc_prefill_gate_params* p, void* stream) {
+  if (!p) return fail(OC_ERR_INVALID, "NULL params");
+  if (!pf_float_dtype(p->dtype)) return fail(OC_ERR_UNSUPPORTED, "prefill dtype %d (float32, float16, bfloat16)",
+                                             p->dtype);
+  if (p->head_dim != 64 && p->head_dim != 128) return fail(OC_ERR_UNSUPPORTED, "head_dim %d (64 or 128)", p->head_dim);
+  if (p->batch < 0 || p->num_q_heads < 0 || p->num_kv_heads < 1 || p->q_len < 1 || p->kv_len < 0)
+    return fail(OC_ERR_INVALID, "bad sizes");
+  if (p->num_q_heads % p->num_kv_heads) return fail(OC_ERR_INVALID, "num_q_heads %d not a multiple of num_kv_heads %d",
+                                                    p->num_q_heads, p->num_kv_heads);
+  const int T = p->kv_len / 64;
+  if (p->batch == 0 || p->num_q_heads == 0 || T == 0) return OC_OK;
+  if (!p->q || !p->k || !p->q_norms || !p->k_norms || !p->mask) return fail(OC_ERR_INVALID, "NULL pointer");
+  const int es = p->dtype == OC_F32 ? 4 : 2;
+  const int64_t strides[] = {p->q_stride_b, p->q_stride_h, p->q_stride_s, p->k_stride_b, p->k_stride_h, p->k_stride_s};
+  for (int64_t st : strides)
+    if ((st * es) % 16) return fail(OC_ERR_INVALID, "q/k strides must be multiples of 16 bytes");
+  if (((uintptr_t)p->q | (uintptr_t)p->k) % 16) return fail(OC_ERR_INVALID, "q/k not 16-byte aligned");
+  if (p->k_stride_s * es * 64 > 0x7FFFFFFF) return fail(OC_ERR_UNSUPPORTED, "token stride too large");
+  if (p->cache && p->cache_stride < T) return fail(OC_ERR_INVALID, "norm cache rows of %lld, %d tiles",
+                                                   (long long)p->cache_stride, T);
+  // one workgroup per 4 tiles, and per 64 query rows at the least
+  if ((int64_t)p->batch * p->num_kv_heads * T + (int64_t)p->batch * p->num_q_heads * (p->q_len / 64 + 1) > 0x7FFFFFFF)
+    return fail(OC_ERR_UNSUPPORTED, "too many tiles and query rows");
+  PfGateArgs a{};
+  a.q = (const char*)p->q, a.k = (const char*)p->k;
+  a.q_sb = p->q_stride_b * es, a.q_sh = p->q_stride_h * es, a.q_ss = p->q_stride_s * es;
+  a.k_sb = p->k_stride_b * es, a.k_sh = p->k_stride_h * es, a.k_ss = p->k_stride_s * es;
+  a.B = p->batch, a.Hq = p->num_q_heads, a.Hkv = p->num_kv_heads, a.G = p->num_q_heads / p->num_kv_heads;
+  a.Sq = p->q_len, a.T = T;
+  a.norm_scale = p->norm_scale, a.tau_norm = p->tau_norm;
+  a.qn = p->q_norms, a.kn = p->k_norms, a.mask = p->mask, a.stats = p->gate_stats;
+  a.cache = p->cache, a.cache_stride = p->cache_stride, a.valid = p->valid_tiles;
+  const hipStream_t s = (hipStream_t)stream;
+  const bool d64 = p->head_dim == 64;
+  switch (p->dtype) {
+    case OC_F32: d64 ? launch_prefill_norms<OC_F32, 64>(a, s) : launch_prefill_norms<OC_F32, 128>(a, s); break;
+    case OC_F16: d64 ? launch_prefill_norms<OC_F16, 64>(a, s) : launch_prefill_norms<OC_F16, 128>(a, s); break;
+    default: d64 ? launch_prefill_norms<OC_BF16, 64>(a, s) : launch_prefill_norms<OC_BF16, 128>(a, s); break;
+  }
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return hip_fail(e, "prefill norms launch");
+  hipLaunchKernelGGL(prefill_gate_kernel, dim3((unsigned)(a.B * a.Hkv)), dim3(kSelThreads), 0, s, a);
+  e = hipGetLastError();
+  return e == hipSuccess ? OC_OK : hip_fail(e, "prefill gate launch");
+}
+
+extern "C" size_t oc_prefill_gate_params_bytes(void) { return sizeof(oc_prefill_gate_params); }
 
 // The hook decode's gate launch (oc_hook_decode); q_row_stride in elements.
 __attribute__((visibility("hidden"))) int oc_internal_hook_gate(

@@ -778,6 +778,55 @@ def group_gate(q_norms: torch.Tensor, k_norms: torch.Tensor, num_kv_heads: int, 
     return (mask, gn, st) if want_stats else (mask, gn)
 
 
+def check_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.device:
+    """The device of a prefill's q (B, Hq, Sq, d) and k, v (B, Hkv, Skv, d),
+    after the checks of their shapes and types."""
+    device = require_gpu(q, k, v)
+    if q.dim() != 4 or k.dim() != 4 or v.shape != k.shape:
+        raise ValueError(f"q (B, Hq, Sq, d) and k, v (B, Hkv, Skv, d) expected, got {tuple(q.shape)}, "
+                         f"{tuple(k.shape)}, {tuple(v.shape)}")
+    if k.shape[0] != q.shape[0] or k.shape[3] != q.shape[3] or q.shape[1] % k.shape[1]:
+        raise ValueError(f"k {tuple(k.shape)} does not match q {tuple(q.shape)}")
+    if not (q.dtype == k.dtype == v.dtype):
+        raise TypeError(f"q, k and v must share a dtype ({q.dtype}, {k.dtype}, {v.dtype})")
+    return device
+
+
+def norm_cache_ready(cache: torch.Tensor, valid_tiles: torch.Tensor, device: torch.device) -> bool:
+    """Whether prefill_gate can write a norm cache's rows itself."""
+    return (cache.device == device and cache.dtype == torch.float32 and cache.stride(1) == 1
+            and valid_tiles.device == device and valid_tiles.dtype == torch.int32 and valid_tiles.is_contiguous())
+
+
+def prefill_gate(q: torch.Tensor, k: torch.Tensor, tau_norm: float, norm_scale: float, *,
+                 stats_out: Optional[torch.Tensor] = None, cache: Optional[torch.Tensor] = None,
+                 valid_tiles: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+    """oc_prefill_gate over q (B, Hq, Sq, d) and k (B, Hkv, Skv, d), both as
+    `ready16` gives them: (evict mask uint8 (B, Hkv, T), norm_scale times
+    the band norms float32 (B, Hkv, T)) of the T = Skv // 64 complete
+    tiles.  stats_out: contiguous float32 (B, Hkv, 3) for group_gate's
+    statistics; cache (>= Hkv, >= T) float32 with contiguous rows and
+    valid_tiles int32 take the last batch element's norms."""
+    device = require_gpu(q, k)
+    B, Hq, Sq, d = q.shape
+    Hkv, T = k.shape[1], k.shape[2] // TILE_SIZE
+    p = N.OcPrefillGateParams()
+    p.q, (p.q_stride_b, p.q_stride_h, p.q_stride_s) = q.data_ptr(), q.stride()[:3]
+    p.k, (p.k_stride_b, p.k_stride_h, p.k_stride_s) = k.data_ptr(), k.stride()[:3]
+    p.dtype = dtype_code(q.dtype, "q", allow_fp8=False)
+    p.batch, p.num_q_heads, p.num_kv_heads, p.q_len, p.kv_len, p.head_dim = B, Hq, Hkv, Sq, k.shape[2], d
+    p.norm_scale, p.tau_norm = norm_scale, tau_norm
+    qn = torch.empty((B, Hq, Sq), dtype=torch.float32, device=device)
+    kn = torch.empty((B, Hkv, T), dtype=torch.float32, device=device)
+    mask = torch.empty((B, Hkv, T), dtype=torch.uint8, device=device)
+    p.q_norms, p.k_norms, p.mask, p.gate_stats = qn.data_ptr(), kn.data_ptr(), mask.data_ptr(), _ptr(stats_out)
+    if cache is not None:
+        p.cache, p.cache_stride, p.valid_tiles = cache.data_ptr(), cache.stride(0), _ptr(valid_tiles)
+    with torch.cuda.device(device):
+        N.check("oc_prefill_gate", N.lib().oc_prefill_gate(ctypes.byref(p), ctypes.c_void_p(current_stream(device))))
+    return mask, kn
+
+
 def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, tile_mask: Optional[torch.Tensor] = None,
                       scale: Optional[float] = None, want_entropy: bool = False, split: bool = True
                       ) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
@@ -788,16 +837,9 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, tile
     None).  split: let the library run the longest causal windows as two
     workgroups each when the call fits the device in one round (it then uses
     the stream's workspace)."""
-    device = require_gpu(q, k, v)
-    if q.dim() != 4 or k.dim() != 4 or v.shape != k.shape:
-        raise ValueError(f"q (B, Hq, Sq, d) and k, v (B, Hkv, Skv, d) expected, got {tuple(q.shape)}, "
-                         f"{tuple(k.shape)}, {tuple(v.shape)}")
+    device = check_prefill(q, k, v)
     B, Hq, Sq, d = q.shape
-    if k.shape[0] != B or k.shape[3] != d or Hq % k.shape[1]:
-        raise ValueError(f"k {tuple(k.shape)} does not match q {tuple(q.shape)}")
-    if not (q.dtype == k.dtype == v.dtype):
-        raise TypeError(f"q, k and v must share a dtype ({q.dtype}, {k.dtype}, {v.dtype})")
-    q, k, v = (_ready16(t) for t in (q, k, v))
+    q, k, v = (ready16(t) for t in (q, k, v))
     Hkv, Skv = k.shape[1], k.shape[2]
     out = torch.empty((B, Hq, Sq, d), dtype=q.dtype, device=device)
     ent = torch.empty((B, Hq, Sq), dtype=torch.float32, device=device) if want_entropy else None
@@ -829,7 +871,7 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, tile
     return out, ent
 
 
-def _ready16(t: torch.Tensor) -> torch.Tensor:
+def ready16(t: torch.Tensor) -> torch.Tensor:
     """t itself when its last dimension is contiguous and its base and every
     other stride are 16-byte aligned (the kernels' vector loads), else a
     contiguous copy."""
@@ -854,7 +896,7 @@ def block_spectra(keys: torch.Tensor, q: Optional[torch.Tensor] = None, *, want_
     device = require_gpu(keys) if q is None else require_gpu(keys, q)
     if keys.dim() != 3:
         raise ValueError(f"keys must be (seq_len, num_heads, head_dim), got {tuple(keys.shape)}")
-    keys = _ready16(keys)
+    keys = ready16(keys)
     S, H, d = keys.shape
     nb = S // SPECTRA_BLOCK
     f32 = dict(dtype=torch.float32, device=device)

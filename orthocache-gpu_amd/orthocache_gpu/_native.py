@@ -88,6 +88,18 @@ class OcPrefillParams(ctypes.Structure):
     ]
 
 
+class OcPrefillGateParams(ctypes.Structure):
+    _fields_ = [
+        ("q", _p), ("q_stride_b", _i64), ("q_stride_h", _i64), ("q_stride_s", _i64),
+        ("k", _p), ("k_stride_b", _i64), ("k_stride_h", _i64), ("k_stride_s", _i64),
+        ("dtype", _i32), ("batch", _i32), ("num_q_heads", _i32), ("num_kv_heads", _i32),
+        ("q_len", _i32), ("kv_len", _i32), ("head_dim", _i32), ("norm_scale", ctypes.c_float),
+        ("tau_norm", ctypes.c_double),
+        ("q_norms", _p), ("k_norms", _p), ("mask", _p), ("gate_stats", _p),
+        ("cache", _p), ("cache_stride", _i64), ("valid_tiles", _p),
+    ]
+
+
 class OcSpectraParams(ctypes.Structure):
     _fields_ = [
         ("k", _p), ("dtype", _i32), ("num_blocks", _i32), ("num_heads", _i32), ("head_dim", _i32),
@@ -137,6 +149,8 @@ SIGNATURES = {
     "oc_prefill_attention": (_i32, [ctypes.POINTER(OcPrefillParams), _p]),
     "oc_prefill_workspace_size": (ctypes.c_size_t, [ctypes.POINTER(OcPrefillParams)]),
     "oc_prefill_params_bytes": (ctypes.c_size_t, []),
+    "oc_prefill_gate": (_i32, [ctypes.POINTER(OcPrefillGateParams), _p]),
+    "oc_prefill_gate_params_bytes": (ctypes.c_size_t, []),
     "oc_block_spectra": (_i32, [ctypes.POINTER(OcSpectraParams), _p]),
     "oc_spectra_params_bytes": (ctypes.c_size_t, []),
     "oc_stream_compact": (_i32, [_p, _i32, _p, _p, _p]),
@@ -199,7 +213,9 @@ def lib():
                     "orthocache_gpu: struct layout mismatch between the binding and "
                     f"{LIB_PATH} ({kv_sz.value}/{p_sz.value} vs "
                     f"{ctypes.sizeof(OcKvDesc)}/{ctypes.sizeof(OcDecodeParams)} bytes)")
-            for fn, st in (("oc_prefill_params_bytes", OcPrefillParams), ("oc_spectra_params_bytes", OcSpectraParams),
+            for fn, st in (("oc_prefill_params_bytes", OcPrefillParams),
+                           ("oc_prefill_gate_params_bytes", OcPrefillGateParams),
+                           ("oc_spectra_params_bytes", OcSpectraParams),
                            ("oc_hook_decode_params_bytes", OcHookDecodeParams)):
                 if getattr(handle, fn)() != ctypes.sizeof(st):
                     raise RuntimeError(f"orthocache_gpu: {st.__name__} layout mismatch between the binding and "

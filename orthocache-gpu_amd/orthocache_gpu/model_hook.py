@@ -50,10 +50,8 @@ import torch
 import torch.nn.functional as F
 
 from . import _launch as X
-from . import _native as N
 
 TILE = 64
-_HIGH_BAND = (48, 64)  # (tile_size * 3) // 4 .. tile_size (perplexity_eval.py:441-442)
 _LOW_BAND = 8          # _compute_q_high_norm's default (perplexity_eval.py:547)
 # The hook transforms with its own unnormalised Sylvester H64, entries +-1
 # (perplexity_eval.py:54-64), which is 8 x the W64 = H64 / 8 of the band-norm
@@ -116,26 +114,30 @@ class _Stats(dict):
         super().__init__(*args, **kw)
         self._pending = []
         self._folding = False
-        self._rings = {}  # (device, shape): views of a (_MAX_PENDING,) + shape float32 device ring
+        self._rings = {}  # (device, shape): a (_MAX_PENDING,) + shape float32 device ring, its views made so far
         self._ring_next = 0
 
     def ring_rows(self, device: torch.device, shape: tuple) -> torch.Tensor:
         """float32 device values of one call, of the given shape, to be
         deferred: a slot of a ring that is free again once the pending calls
         are folded (at most _MAX_PENDING of them), so that a call allocates
-        nothing.  The slots' views are made once."""
+        nothing.  A slot's view is made at its first use (all of them at the
+        first call would cost that call 200 us)."""
         if self._ring_next >= self._MAX_PENDING:
             # (only after calls that failed before deferring) no pending call
             # holds a row once the pending calls are folded
             self.fold()
             self._ring_next = 0
         key = (device, shape)
-        views = self._rings.get(key)
-        if views is None:
+        entry = self._rings.get(key)
+        if entry is None:
             ring = torch.empty((self._MAX_PENDING,) + tuple(shape), dtype=torch.float32, device=device)
-            views = self._rings[key] = list(ring.unbind(0))
+            entry = self._rings[key] = (ring, [None] * self._MAX_PENDING)
+        ring, views = entry
         slot = self._ring_next
         self._ring_next += 1
+        if views[slot] is None:
+            views[slot] = ring[slot]
         return views[slot]
 
     _MAX_PENDING = 256  # calls held before a fold (bounds the device tensors kept alive)
@@ -250,56 +252,57 @@ class OrthoCache_GQA_Attention:
         Hkv, Skv = key.shape[1], key.shape[2]
         T = Skv // TILE
         tau = self._tau()
-        # ||(H64 K_t)[48:64]||_F of every complete tile, (B, Hkv, T)
-        kn = torch.empty((B * Hkv, T), dtype=torch.float32, device=key.device)
-        X.band_norms(X.rows_layout(key.reshape(B * Hkv, Skv, d), None), 0, T, _HIGH_BAND, kn)
-        kn = kn.view(B, Hkv, T).mul_(_HOOK_NORM_SCALE)
-        # per q head: lower median over positions of ||q||_2; the group's max
-        med = X.kth_smallest(X.row_norms(query).view(B * Hq, Sq), (Sq - 1) // 2).view(B, Hq)
-        evict, qn = X.group_gate(med, kn, Hkv, G, T, T, tau * TILE * d, N.OC_GROUP_MAX)
+        X.check_prefill(query, key, value)
+        if Hq != Hkv * G:
+            raise ValueError(f"query has {Hq} heads, {Hkv} kv heads x {G} expected")
+        nc = self.norm_cache
+        if nc is not None and (Hkv > nc.num_kv_heads or T > nc.max_tiles):
+            raise IndexError(f"norm cache ({nc.num_kv_heads} heads x {nc.max_tiles} tiles) is smaller than the "
+                             f"prefill ({Hkv} heads x {T} tiles)")
+        query, key, value = (X.ready16(t) for t in (query, key, value))
+        # the norms ||(H64 K_t)[48:64]||_F of every complete tile, per q head
+        # the lower median over positions of ||q||_2, the group's max, the
+        # gate and its statistics, and the norm cache
+        in_kernel = nc is not None and X.norm_cache_ready(nc.cache, nc.valid_tiles, key.device)
+        dev = self.stats.ring_rows(query.device, (B, Hkv, 3))
+        evict, kn = X.prefill_gate(query, key, tau * TILE * d, _HOOK_NORM_SCALE, stats_out=dev,
+                                   cache=nc.cache if in_kernel else None,
+                                   valid_tiles=nc.valid_tiles if in_kernel else None)
         want_entropy = self.governor is not None and hasattr(self.governor, 'set_entropy')
         out, ent = X.prefill_attention(query, key, value, tile_mask=evict, want_entropy=want_entropy)
-        if self.norm_cache is not None:
-            self._store_norms(kn[B - 1], Hkv, T)
+        if nc is not None:
+            if not in_kernel:
+                # the reference's per-batch loop writes cache[kv_h, t] for every batch
+                # element in turn, so the last one's norms remain (perplexity_eval.py:472-477)
+                nc.cache[:Hkv, :T].copy_(kn[B - 1])
+                nc.valid_tiles[:Hkv].clamp_(min=T)
+            nc._populated = True
         self._prefill_tiles = T
-        # per batch element [evicted, max q norm, max k norm, mean entropy], reduced on the GPU
-        zeros = torch.zeros((B,), dtype=torch.float32, device=query.device)
-        dev = torch.stack([
-            evict.view(B, -1).sum(1, dtype=torch.int64).to(torch.float32),
-            qn.amax(1).clamp(min=0.0),
-            kn.reshape(B, -1).amax(1).clamp(min=0.0),
-            ent.view(B, -1).mean(1) if ent is not None else zeros,
-        ])
+        # dev: per (batch element, kv head) [evicted, q norm, max k norm], then
+        # with an entropy governor the batch elements' mean entropies
+        if want_entropy:
+            dev = torch.cat([dev.reshape(-1), ent.view(B, -1).mean(1)])
         stats, gov = self.stats, self.governor
 
         def fold(host):
+            flat = host.reshape(-1)
             for b in range(B):
-                evicted = int(host[0, b])
+                hb = flat[3 * Hkv * b:3 * Hkv * (b + 1)].reshape(Hkv, 3)
+                evicted = int(hb[:, 0].sum())
                 _add(stats, 'total_tiles', Hkv * T)
                 _add(stats, 'evicted_tiles', evicted)
-                _exhaust(stats, float(host[1, b]), float(host[2, b]))
+                _exhaust(stats, float(np.maximum(hb[:, 1].max(), 0.0)), float(np.maximum(hb[:, 2].max(), 0.0)))
                 if gov is not None and Hkv * T > 0:
                     gov.report_layer(evicted / (Hkv * T))
                 if want_entropy:
-                    gov.set_entropy(float(host[3, b]))
-                    _dset(stats, 'entropy', float(host[3, b]))
+                    entropy = float(flat[3 * Hkv * B + b])
+                    gov.set_entropy(entropy)
+                    _dset(stats, 'entropy', entropy)
             _add(stats, 'layers_processed', 1)
         stats.defer(fold, dev)
         if gov is not None:
             stats.fold()
         return out
-
-    def _store_norms(self, kn_last: torch.Tensor, Hkv: int, T: int) -> None:
-        """The reference's per-batch loop writes cache[kv_h, t] for every batch
-        element in turn, so the last one's norms remain (perplexity_eval.py:472-477)."""
-        nc = self.norm_cache
-        if Hkv > nc.num_kv_heads or T > nc.max_tiles:
-            raise IndexError(f"norm cache ({nc.num_kv_heads} heads x {nc.max_tiles} tiles) is smaller than the "
-                             f"prefill ({Hkv} heads x {T} tiles)")
-        nc.cache[:Hkv, :T].copy_(kn_last)
-        nc.valid_tiles[:Hkv].clamp_(min=T)
-        nc._populated = True
-
 
     # ------------------------------------------------------------ decode
 

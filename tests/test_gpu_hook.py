@@ -432,3 +432,58 @@ def test_hook_decode_mixed_dtypes(qd, kd):
     assert stats.view(B, Hkv, 3)[:, :, 0].sum(dim=1).cpu().tolist() == ref["skipped"].tolist()
     o32, _ = X.hook_decode(q.float(), k.float(), v.float(), norms, G, tau * 64 * d, 8)
     assert torch.equal(out, o32.to(TD[qd]))
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("B,Hq,Hkv,d,Sq,Skv", [(1, 8, 2, 128, 1, 64), (2, 4, 4, 64, 33, 130), (1, 5, 1, 128, 257, 300),
+                                               (2, 18, 2, 64, 129, 129), (1, 16, 2, 128, 2049, 2049),
+                                               (1, 2, 1, 64, 16500, 16500)], ids=lambda x: str(x))
+def test_prefill_gate_vs_oracle(dtype, B, Hq, Hkv, d, Sq, Skv):
+    """oc_prefill_gate at its edges: one query row, rows that do not fill a
+    wave's loads, 1 to 9 heads of a group (up to eight are selected at once),
+    and more rows than the selection holds in registers; q is the transposed
+    view a decoder layer passes, K a slice of a longer cache."""
+    from orthocache_gpu import _launch as X
+    G, T = Hq // Hkv, Skv // 64
+    g = torch.Generator().manual_seed(Sq + Hq)
+    q = torch.randn((B, Sq, Hq, d), generator=g).to(TD[dtype]).to(DEV).transpose(1, 2)
+    k = torch.randn((B, Hkv, Skv + 8, d), generator=g).to(TD[dtype]).to(DEV)[:, :, :Skv]
+    kn_ref = O.hook_tile_norms(np64(k))
+    qn_ref = O.torch_lower_median(np.linalg.norm(np64(q), axis=-1)).reshape(B, Hkv, G).max(axis=2)
+    prods = qn_ref[:, :, None] * kn_ref.astype(np.float64)
+    tau_norm = _gap_tau(prods) if prods.size >= 4 else float(prods.mean())
+    st = torch.full((B, Hkv, 3), -1.0, device=DEV)
+    cache = torch.full((Hkv + 1, T + 2), -5.0, device=DEV)
+    valid = torch.tensor([0] + [T + 1] * Hkv, dtype=torch.int32, device=DEV)
+    print(f"prefill gate {dtype} B={B} Hq={Hq} Hkv={Hkv} d={d} Sq={Sq} Skv={Skv}", flush=True)
+    mask, kn = X.prefill_gate(q, k, tau_norm, 8.0, stats_out=st, cache=cache, valid_tiles=valid)
+    # sums of 16 d squares, and of d, in float32
+    np.testing.assert_allclose(np64(kn), kn_ref, rtol=4 * 2.0 ** -23)
+    st = st.cpu().numpy()
+    np.testing.assert_allclose(st[:, :, 1], qn_ref, rtol=8 * 2.0 ** -23)
+    evict = prods <= tau_norm
+    assert np.array_equal(mask.cpu().numpy().astype(bool), evict)
+    assert np.array_equal(st[:, :, 0], evict.sum(axis=2)) and np.array_equal(st[:, :, 2], kn.cpu().numpy().max(axis=2))
+    # the last batch element's norms, nothing beside them; counts raised only
+    assert torch.equal(cache[:Hkv, :T], kn[B - 1])
+    assert (cache[Hkv:] == -5).all() and (cache[:, T:] == -5).all()
+    assert valid.cpu().tolist() == [T] + [T + 1] * Hkv
+
+
+def test_selection_of_clustered_long_and_odd_rows():
+    """Rows longer than the selection holds in registers, rows whose values
+    share all or nearly all bits, and rows of the full float range with NaN
+    (which sorts last) and infinity: the value is exact."""
+    from orthocache_gpu import _launch as X
+    g = torch.Generator().manual_seed(6)
+    for n in (16384, 16385, 50000):
+        base = torch.randn((1, n), generator=g).abs()
+        rows = [base, base * 1e-30, base.exp() ** 8, torch.full((1, n), 11.25), 11.0 + base * 1e-6, base.clone()]
+        rows[2][0, ::7] = 0.0
+        rows[5][0, 3::11] = float("nan")
+        rows[5][0, 5::13] = float("inf")
+        x = torch.cat(rows)
+        srt = np.sort(x.numpy(), axis=1)  # numpy sorts NaN last
+        for k in (0, 1, (n - 1) // 2, n - 1):
+            sel = X.kth_smallest(x.to(DEV), k).cpu().numpy()
+            assert np.array_equal(sel, srt[:, k], equal_nan=True), (n, k)
