@@ -373,6 +373,43 @@ size_t oc_prefill_workspace_size(const oc_prefill_params* p);
 size_t oc_prefill_params_bytes(void);
 
 /*
+ * oc_attend -- softmax(q k^T * scale) v of every query over every token of
+ * the retained 64-token tiles (no causal limit): tile t is attended when
+ * tile_mask[h * tile_mask_stride_h + t] != 0, or always without a mask; a
+ * query with no tile gets zeros.  float32 accumulation; out in out_dtype.
+ * The compact pipeline's attention and its dense path for a chunk of
+ * queries (adaptive_attention.py:46-91, pipeline.py:558-568).  dtype
+ * F32/F16/BF16, head_dim 64 or 128, q/k/v rows 16-byte aligned, kv_len up to
+ * 1M tokens.
+ */
+typedef struct oc_attend_params {
+  const void* q;                  /* (q_len, num_heads, head_dim) */
+  int64_t q_stride_s, q_stride_h; /* elements; head_dim contiguous */
+  const void* k;                  /* (kv_len, num_heads, head_dim) */
+  int64_t k_stride_s, k_stride_h;
+  const void* v;
+  int64_t v_stride_s, v_stride_h;
+  void* out;                      /* (q_len, num_heads, head_dim), out_stride_s = num_heads * out_stride_h */
+  int64_t out_stride_s, out_stride_h;
+  int32_t dtype, out_dtype;       /* of q, k and v; of out */
+  int32_t num_heads, q_len, kv_len, head_dim;
+  const uint8_t* tile_mask;       /* (num_heads, >= kv_len / 64 rounded up) or NULL */
+  int64_t tile_mask_stride_h;     /* 0: one row for all heads */
+  float scale;
+  int32_t num_splits;             /* shares of a head's tiles; 0: chosen from the sizes */
+  void* workspace;                /* >= oc_attend_workspace_size(p) bytes; its first 64 KiB are not touched */
+  size_t workspace_bytes;
+} oc_attend_params;
+
+int oc_attend(const oc_attend_params* p, void* stream);
+
+/* bytes of workspace oc_attend needs (0: none) */
+size_t oc_attend_workspace_size(const oc_attend_params* p);
+
+/* sizeof(oc_attend_params) as compiled, for binding checks */
+size_t oc_attend_params_bytes(void);
+
+/*
  * oc_prefill_gate -- the tile gate of the hook's prefill (perplexity_eval.py:
  * 441-491) in two launches: q_norms = ||q[b, h, s]||_2 of every query row,
  * k_norms = norm_scale * ||(W64 K_t)[48:64]||_F of every complete tile t <

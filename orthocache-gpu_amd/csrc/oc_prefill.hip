@@ -350,13 +350,14 @@ __device__ __forceinline__ void pf_logits(const PfQ<DT, D>& q, const char* sk, i
 // output column 16nc + 4r + i of query x in lane 16r + x.  16-bit: per
 // 32-token block j, A = V^T read with ds_read_b64_tr_b16 from the permuted
 // rows (lane group g gets tokens 32j + 4g + b and 32j + 16 + 4g + b), B =
-// the lane's own eight probabilities c[2j][b], c[2j + 1][b]: float16 rounds
-// them once (relative error at most 2^-12); bfloat16 sends a 16-bit high
-// part plus the 16-bit rounding of the remainder (two instructions), since
-// one rounding (2^-9) moves short causal rows past the output tolerance.
+// the lane's own eight probabilities c[2j][b], c[2j + 1][b].  HILO sends a
+// 16-bit high part plus the 16-bit rounding of the remainder (two
+// instructions); without it they are rounded once, which the causal kernel
+// does for float16 (relative error at most 2^-12): in bfloat16 one rounding
+// (2^-9) moves short causal rows past the output tolerance.
 // float32: 16x16x4 steps over (tb, i), A = V[16tb + 4r + i][16nc + x], B =
 // c[tb][i], exact.
-template <int DT, int D>
+template <int DT, int D, bool HILO = DT == OC_BF16>
 __device__ __forceinline__ void pf_pv(f32x4 (&acc)[D / 16], const f32x4 (&c)[4], const char* svb, int lane) {
   const int x = lane & 15;
   const int kg = lane >> 4;
@@ -386,6 +387,7 @@ __device__ __forceinline__ void pf_pv(f32x4 (&acc)[D / 16], const f32x4 (&c)[4],
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         if constexpr (DT == OC_BF16) {
+          static_assert(HILO, "bfloat16 probabilities are split");
           const __bf16 h0 = (__bf16)pv[2 * e], h1 = (__bf16)pv[2 * e + 1];
           const __bf16 l0 = (__bf16)(pv[2 * e] - (float)h0), l1 = (__bf16)(pv[2 * e + 1] - (float)h1);
           bhi[e] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
@@ -393,6 +395,10 @@ __device__ __forceinline__ void pf_pv(f32x4 (&acc)[D / 16], const f32x4 (&c)[4],
         } else {
           const _Float16 h0 = (_Float16)pv[2 * e], h1 = (_Float16)pv[2 * e + 1];
           bhi[e] = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
+          if constexpr (HILO) {
+            const _Float16 l0 = (_Float16)(pv[2 * e] - (float)h0), l1 = (_Float16)(pv[2 * e + 1] - (float)h1);
+            blo[e] = (uint32_t)__builtin_bit_cast(uint16_t, l0) | ((uint32_t)__builtin_bit_cast(uint16_t, l1) << 16);
+          }
         }
       }
       // lane x of group kg reads rows 32j + 8kg + 4h + x/4 (h = 0, 1), column
@@ -423,7 +429,7 @@ __device__ __forceinline__ void pf_pv(f32x4 (&acc)[D / 16], const f32x4 (&c)[4],
 #pragma unroll
         for (int g = 0; g < kPfPvGroup; ++g) {
           acc[n0 + g] = mfma_qk<DT>(av[g], bhi, acc[n0 + g]);
-          if constexpr (DT == OC_BF16) acc[n0 + g] = mfma_qk<DT>(av[g], blo, acc[n0 + g]);
+          if constexpr (HILO) acc[n0 + g] = mfma_qk<DT>(av[g], blo, acc[n0 + g]);
         }
       }
     }
@@ -657,6 +663,202 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(DT =
       a.entropy[((int64_t)b * a.Hq + h) * a.Sq + qpos_o] = H;
     }
   }
+}
+
+// ------------------------------------------------ attention of a query block
+//
+// Every query of a block of up to 128 attends every token of the tiles that
+// a mask retains (no causal limit): the compact pipeline's attention and the
+// dense mode with more than a few queries.  It is the prefill kernel's tile
+// step (K and V of a tile staged once in LDS for eight waves of 16 queries)
+// over one share of the head's retained tiles per workgroup; the shares'
+// states are combined by the merge kernel.  Bound by the K/V bytes while the
+// queries of a head fit one block.  70 queries, 32 heads of 128, half of 8192
+// tokens retained (67 MB, bfloat16): 26 us and 5.8 us for the merge; the decode
+// kernels, which read the tiles again for every eight queries, took 88 us and
+// four copies of q and of the output around them.
+
+constexpr int kAtMaxWords = 256;  // 64-tile words of the retained-tile bits (rows of up to 1M tokens)
+
+struct AttendArgs {
+  const char* q;
+  const char* k;
+  const char* v;
+  char* out;
+  int64_t q_ss, q_sh, k_ss, k_sh, v_ss, v_sh, o_ss, o_sh;  // byte strides (position, head)
+  int32_t H, Sq, Skv, T, P, qblocks, out_dtype;            // T: tiles, a partial last one included
+  const uint8_t* mask;  // (H, >= Skv / 64) attend flags or null (every tile)
+  int64_t m_sh;
+  float scale;
+  float* pm;  // partial states of row s * H + h, share g: at row * P + g
+  float* pl;
+  float* pacc;
+};
+
+template <int DT, int D>
+__global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(DT == OC_F32 && D == 128 ? 1 : 4))) void attend_kernel(
+    const AttendArgs a) {
+  using L = PfTile<DT, D>;
+  __shared__ __attribute__((aligned(16))) char sh[L::LDS];
+  __shared__ uint64_t bits[kAtMaxWords + 1];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  // the query blocks of one (head, share) read the same tiles: workgroup i
+  // runs on XCD i mod 8, so they are numbered eight apart
+  const int pairs = a.H * a.P;
+  int pair, qb;
+  if (pairs % 8 == 0) {
+    const int j = blockIdx.x / 8;
+    qb = j % a.qblocks;
+    pair = j / a.qblocks * 8 + blockIdx.x % 8;
+  } else {
+    pair = blockIdx.x % pairs;
+    qb = blockIdx.x / pairs;
+  }
+  const int h = pair / a.P, g = pair % a.P;
+  const int pos0 = qb * kPfRows + 16 * wave;
+  const int x = lane & 15, r = lane >> 4;
+  const float scale2 = a.scale * 1.4426950408889634f;  // log2 e
+
+  PrefillArgs pa;  // what the tile staging and the q load read
+  pa.q_ss = a.q_ss, pa.Sq = a.Sq, pa.Skv = a.Skv, pa.k_ss = a.k_ss, pa.v_ss = a.v_ss;
+  PfQ<DT, D> q;
+  pf_load_q<DT, D>(pa, a.q + (int64_t)h * a.q_sh, pos0, lane, q);
+  const char* kh = a.k + (int64_t)h * a.k_sh;
+  const char* vh = a.v + (int64_t)h * a.v_sh;
+
+  // the share: retained tiles of ranks [n0, n1) (all tiles without a mask),
+  // walked through the words of the retained-tile bits
+  const int words = (a.T + 63) / 64;
+  for (int w = wave; w < words; w += kPfWaves) {
+    const int t = 64 * w + lane;
+    const uint64_t b =
+        __builtin_amdgcn_ballot_w64(t < a.T && (!a.mask || a.mask[(int64_t)h * a.m_sh + min(t, a.T - 1)] != 0));
+    if (lane == 0) bits[w] = b;
+  }
+  if (tid == 0) bits[words] = 0;  // read past the last tile, never used
+  __syncthreads();
+  int kept = 0;
+  for (int w0 = 0; w0 < words; w0 += 64) kept += (int)wave_sum(w0 + lane < words ? (float)__popcll(bits[w0 + lane]) : 0.f);
+  const int n0 = (int)((int64_t)kept * g / a.P), n1 = (int)((int64_t)kept * (g + 1) / a.P);
+  int word = 0, skip = n0;
+  uint64_t cur = bits[0];
+  while (word < words && skip >= __popcll(cur)) {
+    skip -= __popcll(cur);
+    cur = bits[++word];
+  }
+  for (; skip > 0; --skip) cur &= cur - 1;
+  int left = n1 - n0;
+  // the next tile of the share, or -1 (uniform over the workgroup)
+  auto next = [&]() {
+    if (left == 0) return -1;
+    --left;
+    while (cur == 0) cur = bits[++word];
+    const int t = 64 * word + __builtin_ctzll(cur);
+    cur &= cur - 1;
+    return __builtin_amdgcn_readfirstlane(t);
+  };
+
+  const bool active = pos0 < a.Sq;
+  PfState st{kM0, 0.f, 0.f, 0};
+  f32x4 accp[D / 16];
+#pragma unroll
+  for (int nc = 0; nc < D / 16; ++nc) accp[nc] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto stage_k = [&](int s) { return sh + s * 2 * L::KV; };
+  auto stage_v = [&](int s) { return sh + s * 2 * L::KV + L::KV; };
+  // 16-bit probabilities always as two parts, as the decode kernels' p . V
+  auto tile = [&](int t, const char* __restrict__ ck, const char* __restrict__ cv) {
+    f32x4 c[4];
+    pf_logits<DT, D>(q, ck, lane, c);
+    pf_softmax<D, false>(st, accp, c, scale2, a.Skv, t * 64, t * 64 + 64 <= a.Skv, lane);
+    pf_pv<DT, D, true>(accp, c, cv, lane);
+  };
+  int t = next();
+  if constexpr (L::STAGES == 2) {
+    // as in the prefill kernel: the next tile goes straight to the other
+    // stage while this one is used; the stages are restrict parameters
+    if (t >= 0) pf_fetch_lds<DT, D>(pa, kh, vh, t, tid, stage_k(0), stage_v(0));
+    __builtin_amdgcn_s_waitcnt(0);
+    int s = 0;
+    auto step = [&](int tn, char* __restrict__ nk, char* __restrict__ nv, const char* __restrict__ ck,
+                    const char* __restrict__ cv) {
+      if (tn >= 0) pf_fetch_lds<DT, D>(pa, kh, vh, tn, tid, nk, nv);
+      if (active) tile(t, ck, cv);
+    };
+    while (t >= 0) {
+      __syncthreads();  // stage s is complete; every wave is done with stage s ^ 1
+      const int tn = next();
+      step(tn, stage_k(1 - s), stage_v(1 - s), stage_k(s), stage_v(s));
+      __builtin_amdgcn_s_waitcnt(0);
+      s = 1 - s;
+      t = tn;
+    }
+  } else {
+    PfStage<DT, D> reg;
+    if (t >= 0) {
+      pf_fetch<DT, D>(pa, kh, vh, t, tid, reg);
+      pf_stash<DT, D>(reg, tid, stage_k(0), stage_v(0));
+    }
+    while (t >= 0) {
+      __syncthreads();  // the stage is complete
+      const int tn = next();
+      if (tn >= 0) pf_fetch<DT, D>(pa, kh, vh, tn, tid, reg);  // in flight during this tile
+      if (active) tile(t, stage_k(0), stage_v(0));
+      __syncthreads();  // the stage is free again
+      if (tn >= 0) pf_stash<DT, D>(reg, tid, stage_k(0), stage_v(0));
+      t = tn;
+    }
+  }
+  const int s = pos0 + x;
+  if (s >= a.Sq) return;
+  // sums over the query's four lanes (lane 16r + x holds columns 16nc + 4r .. + 4)
+  float l = st.l;
+  l += xpair<16>(l);
+  l += xpair<32>(l);
+  if (a.P == 1) {
+    const float inv = 1.f / fmaxf(l, 1e-9f);
+    char* orow = a.out + (int64_t)h * a.o_sh + (int64_t)s * a.o_ss;
+    const int oes = a.out_dtype == OC_F32 ? 4 : 2;
+#pragma unroll
+    for (int nc = 0; nc < D / 16; ++nc)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) store_scalar(orow + oes * (16 * nc + 4 * r + e), a.out_dtype, accp[nc][e] * inv);
+    return;
+  }
+  const int64_t o = ((int64_t)s * a.H + h) * a.P + g;
+  if (r == 0) {
+    a.pm[o] = st.m * 0.6931471805599453f;  // the merge's weights are e^(m - max)
+    a.pl[o] = l;
+  }
+#pragma unroll
+  for (int nc = 0; nc < D / 16; ++nc)
+    *reinterpret_cast<float4*>(a.pacc + o * D + 16 * nc + 4 * r) =
+        float4{accp[nc][0], accp[nc][1], accp[nc][2], accp[nc][3]};
+}
+
+template <int DT>
+void launch_attend(const AttendArgs& a, int d, unsigned blocks, hipStream_t s) {
+  if (d == 64) hipLaunchKernelGGL((attend_kernel<DT, 64>), dim3(blocks), dim3(kPfThreads), 0, s, a);
+  else hipLaunchKernelGGL((attend_kernel<DT, 128>), dim3(blocks), dim3(kPfThreads), 0, s, a);
+}
+
+// Shares per head: about kAtPerCu workgroups per CU, and at least kAtMinTiles
+// tiles a share (before the mask).  32 heads of 128 over 32768 tokens, half
+// retained, nine queries: 70 us at one per CU (8 shares), 60 at two, 69 at
+// four; 8 heads over 16384 tokens: 21, 16.5 at two (32 shares and more).
+constexpr int kAtPerCu = 2, kAtMinTiles = 4;
+
+int attend_shares(const oc_attend_params* p) {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    cus = 256;
+  const int64_t blocks = (int64_t)p->num_heads * ((p->q_len + kPfRows - 1) / kPfRows);
+  const int64_t tiles = (p->kv_len + 63) / 64;
+  if (p->num_splits > 0) return (int)std::max<int64_t>(1, std::min<int64_t>({p->num_splits, tiles, 8192}));
+  if (blocks == 0) return 1;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(kAtPerCu * cus / blocks, tiles / kAtMinTiles));
 }
 
 // ------------------------------------------------------------ gate helpers
@@ -1348,6 +1550,81 @@ extern "C" size_t oc_prefill_workspace_size(const oc_prefill_params* p) {
   PfPlan pl;
   return pf_plan(p, &pl) ? kPfCounterBytes + pl.part_bytes + 256 : 0;
 }
+
+static int attend_check(const oc_attend_params* p) {
+  if (!p) return fail(OC_ERR_INVALID, "NULL params");
+  if (!pf_float_dtype(p->dtype) || !pf_float_dtype(p->out_dtype))
+    return fail(OC_ERR_UNSUPPORTED, "attention dtypes %d, %d (float32, float16, bfloat16)", p->dtype, p->out_dtype);
+  if (p->head_dim != 64 && p->head_dim != 128) return fail(OC_ERR_UNSUPPORTED, "head_dim %d (64 or 128)", p->head_dim);
+  if (p->num_heads < 0 || p->q_len < 0 || p->kv_len < 0 || p->num_splits < 0) return fail(OC_ERR_INVALID, "bad sizes");
+  if (p->kv_len > 64 * 64 * kAtMaxWords)
+    return fail(OC_ERR_UNSUPPORTED, "kv_len %d over %d", p->kv_len, 64 * 64 * kAtMaxWords);
+  if ((int64_t)p->num_heads * ((p->q_len + kPfRows - 1) / kPfRows) > 0x7FFFFFFF / 8192)
+    return fail(OC_ERR_UNSUPPORTED, "too many query blocks");
+  return OC_OK;
+}
+
+// [merge counters of the decode calls that share the workspace] [acc] [m] [l]
+extern "C" size_t oc_attend_workspace_size(const oc_attend_params* p) {
+  if (attend_check(p)) return 0;
+  const int P = attend_shares(p);
+  if (P == 1) return 0;
+  return kPfCounterBytes + 256 + (size_t)p->num_heads * p->q_len * P * (p->head_dim + 2) * sizeof(float);
+}
+
+extern "C" int oc_attend(const oc_attend_params* p, void* stream) {
+  int rc = attend_check(p);
+  if (rc) return rc;
+  if (p->num_heads == 0 || p->q_len == 0) return OC_OK;
+  if (!p->q || !p->k || !p->v || !p->out) return fail(OC_ERR_INVALID, "NULL tensor pointer");
+  const int es = p->dtype == OC_F32 ? 4 : 2, oes = p->out_dtype == OC_F32 ? 4 : 2;
+  const int64_t strides[] = {p->q_stride_s, p->q_stride_h, p->k_stride_s, p->k_stride_h, p->v_stride_s, p->v_stride_h};
+  for (int64_t st : strides)
+    if ((st * es) % 16) return fail(OC_ERR_INVALID, "q/k/v strides must be multiples of 16 bytes");
+  if (((uintptr_t)p->q | (uintptr_t)p->k | (uintptr_t)p->v) % 16) return fail(OC_ERR_INVALID, "q/k/v not 16-byte aligned");
+  if ((uintptr_t)p->out % oes) return fail(OC_ERR_INVALID, "out not aligned to its elements");
+  if (p->k_stride_s * es * 64 > 0x7FFFFFFF || p->v_stride_s * es * 64 > 0x7FFFFFFF)
+    return fail(OC_ERR_UNSUPPORTED, "token stride too large");
+  if (p->k_stride_s < p->head_dim || p->v_stride_s < p->head_dim)
+    return fail(OC_ERR_INVALID, "token stride smaller than head_dim");
+  // the merged rows are q_len * num_heads rows of one stride
+  if (p->out_stride_s != p->out_stride_h * p->num_heads)
+    return fail(OC_ERR_INVALID, "out rows (position, head) must have one stride");
+  AttendArgs a{};
+  a.q = (const char*)p->q, a.k = (const char*)p->k, a.v = (const char*)p->v, a.out = (char*)p->out;
+  a.q_ss = p->q_stride_s * es, a.q_sh = p->q_stride_h * es;
+  a.k_ss = p->k_stride_s * es, a.k_sh = p->k_stride_h * es;
+  a.v_ss = p->v_stride_s * es, a.v_sh = p->v_stride_h * es;
+  a.o_ss = p->out_stride_s * oes, a.o_sh = p->out_stride_h * oes;
+  a.H = p->num_heads, a.Sq = p->q_len, a.Skv = p->kv_len, a.T = (p->kv_len + 63) / 64;
+  a.qblocks = (p->q_len + kPfRows - 1) / kPfRows;
+  a.P = attend_shares(p);
+  a.out_dtype = p->out_dtype;
+  a.mask = p->tile_mask, a.m_sh = p->tile_mask_stride_h;
+  a.scale = p->scale;
+  const int64_t rows = (int64_t)a.Sq * a.H;
+  if (a.P > 1) {
+    const size_t need = oc_attend_workspace_size(p);
+    if (!p->workspace || p->workspace_bytes < need)
+      return fail(OC_ERR_WORKSPACE, "attention workspace of %zu bytes needed, %zu given", need, p->workspace_bytes);
+    a.pacc = (float*)((((uintptr_t)p->workspace + 255) & ~(uintptr_t)255) + kPfCounterBytes);
+    a.pm = a.pacc + rows * a.P * p->head_dim;
+    a.pl = a.pm + rows * a.P;
+  }
+  const unsigned blocks = (unsigned)((int64_t)a.H * a.P * a.qblocks);
+  const hipStream_t s = (hipStream_t)stream;
+  switch (p->dtype) {
+    case OC_F32: launch_attend<OC_F32>(a, p->head_dim, blocks, s); break;
+    case OC_F16: launch_attend<OC_F16>(a, p->head_dim, blocks, s); break;
+    default: launch_attend<OC_BF16>(a, p->head_dim, blocks, s); break;
+  }
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return hip_fail(e, "attention launch");
+  if (a.P == 1) return OC_OK;
+  return oc_lse_merge(a.pm, a.pl, a.pacc, (int32_t)rows, a.P, p->head_dim, p->out, p->out_dtype, p->out_stride_h, stream);
+}
+
+extern "C" size_t oc_attend_params_bytes(void) { return sizeof(oc_attend_params); }
 
 extern "C" int oc_row_norms(const void* x, int32_t dtype, int64_t n0, int64_t n1, int64_t n2, int64_t stride0,
                             int64_t stride1, int64_t stride2, int32_t head_dim, int32_t low_band, float* out,

@@ -778,6 +778,55 @@ def group_gate(q_norms: torch.Tensor, k_norms: torch.Tensor, num_kv_heads: int, 
     return (mask, gn, st) if want_stats else (mask, gn)
 
 
+def attend_takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
+    """Whether q (Sq, H, d) over k, v (S, H, d) goes to oc_attend rather than
+    to the decode kernels: one float type, head_dim 64 or 128, at most 1M
+    tokens, and more than one query in 16 bits, more than eight in float32.
+    Half the tiles retained, 32 heads of 128, decode against oc_attend in us:
+    bfloat16 over 32768 tokens 54 / 60 for one query, 63 / 60 for two, 96 / 61
+    for nine and 313 / 75 for 70; float32 over 16384 tokens 81 / 102 for eight
+    and 123 / 102 for nine (the decode holds a float32 tile in registers, the
+    query block stages it through LDS).  Eight is what the decode kernels take
+    in one pass over a head's K and V."""
+    few = 8 if q.dtype == torch.float32 else 1
+    return (q.shape[0] > few and q.dtype == k.dtype == v.dtype and q.shape[2] in (64, 128)
+            and q.dtype in (torch.float32, torch.float16, torch.bfloat16) and 0 < k.shape[0] <= 1 << 20
+            and q.shape[1:] == k.shape[1:] and k.shape == v.shape)
+
+
+def attend(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out_dtype: torch.dtype, *,
+           tile_mask: Optional[torch.Tensor] = None, num_splits: int = 0) -> torch.Tensor:
+    """oc_attend of q (Sq, H, d) over k, v (S, H, d) (what attend_takes
+    takes): (Sq, H, d) in out_dtype.  tile_mask: uint8 (>= S // 64 rounded
+    up,), shared by the heads, 1 = attend."""
+    device = require_gpu(q, k, v)
+    Sq, H, d = q.shape
+    q, k, v = (ready16(t) for t in (q, k, v))
+    out = torch.empty((Sq, H, d), dtype=out_dtype, device=device)
+    p = N.OcAttendParams()
+    p.q, (p.q_stride_s, p.q_stride_h) = q.data_ptr(), q.stride()[:2]
+    p.k, (p.k_stride_s, p.k_stride_h) = k.data_ptr(), k.stride()[:2]
+    p.v, (p.v_stride_s, p.v_stride_h) = v.data_ptr(), v.stride()[:2]
+    p.out, p.out_stride_s, p.out_stride_h = out.data_ptr(), H * d, d
+    p.dtype, p.out_dtype = dtype_code(q.dtype, "q", allow_fp8=False), dtype_code(out_dtype, "out", allow_fp8=False)
+    p.num_heads, p.q_len, p.kv_len, p.head_dim = H, Sq, k.shape[0], d
+    p.scale, p.num_splits = 1.0 / d ** 0.5, num_splits
+    if tile_mask is not None:
+        if (tile_mask.dtype != torch.uint8 or tile_mask.dim() != 1 or not tile_mask.is_contiguous()
+                or tile_mask.device != device or tile_mask.numel() * TILE_SIZE < k.shape[0]):
+            raise ValueError(f"tile_mask must be a contiguous uint8 vector of every tile on {device}")
+        p.tile_mask = tile_mask.data_ptr()
+    lib = N.lib()
+    stream = current_stream(device)
+    with torch.cuda.device(device):
+        need = lib.oc_attend_workspace_size(ctypes.byref(p))
+        if need:
+            ws = workspace(device, stream, need)
+            p.workspace, p.workspace_bytes = ws.data_ptr(), ws.numel()
+        N.check("oc_attend", lib.oc_attend(ctypes.byref(p), ctypes.c_void_p(stream)))
+    return out
+
+
 def check_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.device:
     """The device of a prefill's q (B, Hq, Sq, d) and k, v (B, Hkv, Skv, d),
     after the checks of their shapes and types."""

@@ -88,6 +88,19 @@ class OcPrefillParams(ctypes.Structure):
     ]
 
 
+class OcAttendParams(ctypes.Structure):
+    _fields_ = [
+        ("q", _p), ("q_stride_s", _i64), ("q_stride_h", _i64),
+        ("k", _p), ("k_stride_s", _i64), ("k_stride_h", _i64),
+        ("v", _p), ("v_stride_s", _i64), ("v_stride_h", _i64),
+        ("out", _p), ("out_stride_s", _i64), ("out_stride_h", _i64),
+        ("dtype", _i32), ("out_dtype", _i32),
+        ("num_heads", _i32), ("q_len", _i32), ("kv_len", _i32), ("head_dim", _i32),
+        ("tile_mask", _p), ("tile_mask_stride_h", _i64), ("scale", ctypes.c_float), ("num_splits", _i32),
+        ("workspace", _p), ("workspace_bytes", ctypes.c_size_t),
+    ]
+
+
 class OcPrefillGateParams(ctypes.Structure):
     _fields_ = [
         ("q", _p), ("q_stride_b", _i64), ("q_stride_h", _i64), ("q_stride_s", _i64),
@@ -149,6 +162,9 @@ SIGNATURES = {
     "oc_prefill_attention": (_i32, [ctypes.POINTER(OcPrefillParams), _p]),
     "oc_prefill_workspace_size": (ctypes.c_size_t, [ctypes.POINTER(OcPrefillParams)]),
     "oc_prefill_params_bytes": (ctypes.c_size_t, []),
+    "oc_attend": (_i32, [ctypes.POINTER(OcAttendParams), _p]),
+    "oc_attend_workspace_size": (ctypes.c_size_t, [ctypes.POINTER(OcAttendParams)]),
+    "oc_attend_params_bytes": (ctypes.c_size_t, []),
     "oc_prefill_gate": (_i32, [ctypes.POINTER(OcPrefillGateParams), _p]),
     "oc_prefill_gate_params_bytes": (ctypes.c_size_t, []),
     "oc_block_spectra": (_i32, [ctypes.POINTER(OcSpectraParams), _p]),
@@ -215,6 +231,7 @@ def lib():
                     f"{ctypes.sizeof(OcKvDesc)}/{ctypes.sizeof(OcDecodeParams)} bytes)")
             for fn, st in (("oc_prefill_params_bytes", OcPrefillParams),
                            ("oc_prefill_gate_params_bytes", OcPrefillGateParams),
+                           ("oc_attend_params_bytes", OcAttendParams),
                            ("oc_spectra_params_bytes", OcSpectraParams),
                            ("oc_hook_decode_params_bytes", OcHookDecodeParams)):
                 if getattr(handle, fn)() != ctypes.sizeof(st):

@@ -5,8 +5,9 @@ The reference compacts the block list (stream_compact) and loops over the
 active blocks with an online softmax per head; here the block mask becomes
 a 64-token tile mask and the split-K decode kernel (oc_decode with
 OC_GATE_MASK) attends exactly the retained tiles, never reading an evicted
-block's K or V.  Every query of q attends every retained key (no causal
-mask), as in the reference; the output is bfloat16, as there.
+block's K or V; more than a few queries go to the query-block kernel
+(oc_attend) on the same mask.  Every query of q attends every retained key
+(no causal mask), as in the reference; the output is bfloat16, as there.
 """
 
 from __future__ import annotations
@@ -60,9 +61,15 @@ def attend_tiles(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, 
     seq_q, nh, hd = q.shape
     if tokens > k_cache.shape[0] or tokens % X.TILE_SIZE:
         raise ValueError(f"{tokens} tokens: more than the cache holds or not whole tiles")
+    if X.attend_takes(q, k_cache[:tokens], v_cache[:tokens]):
+        return X.attend(q, k_cache[:tokens], v_cache[:tokens], torch.bfloat16, tile_mask=tile_mask.reshape(-1))
     kv = X.rows_layout(k_cache[:tokens].permute(1, 0, 2), v_cache[:tokens].permute(1, 0, 2))
     tm = tile_mask.reshape(1, -1).expand(nh, -1)
     out = torch.empty((seq_q, nh, hd), dtype=torch.bfloat16, device=q.device)
+    if seq_q == 1:  # the decode's output rows are this call's
+        X.decode(kv, q[0], 1, gate=N.OC_GATE_MASK, threshold=0.0, mode=N.OC_MODE_CACHED, out_dtype=torch.bfloat16,
+                 tile_mask=tm, out=out[0])
+        return out
     for s0 in range(0, seq_q, _Q_CHUNK):
         qq = q[s0:s0 + _Q_CHUNK].permute(1, 0, 2).contiguous()  # (heads, g, d)
         g = qq.shape[1]

@@ -175,9 +175,12 @@ def get_crossover_threshold(device=None) -> int:
 
 def _dense_attention(q: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, head_dim: int) -> torch.Tensor:
     """Dense softmax attention of every query token over every key
-    (pipeline.py:558-568), on the HIP decode kernel with the gate off.
+    (pipeline.py:558-568), on the HIP decode kernel with the gate off, or
+    the query-block kernel for more than a few queries.
     q (Sq, H, d), keys/values (S, H, d) -> (Sq, H, d) in q.dtype."""
     sq, h, d = q.shape
+    if X.attend_takes(q, keys, values):
+        return X.attend(q, keys, values, q.dtype)
     s_len = keys.shape[0]
     k_rows = keys.permute(1, 0, 2)
     v_rows = values.permute(1, 0, 2)

@@ -296,3 +296,49 @@ def test_orthocache_attention_batched():
         assert torch.equal(out[b], one)
     zero, st0 = orthocache_attention_batched(q, k, v, torch.zeros(3, dtype=torch.bool, device=DEV))
     assert not zero.any() and st0["num_active"] == 0
+
+
+@pytest.mark.parametrize("dtype,d", [("f32", 64), ("f32", 128), ("f16", 64), ("f16", 128), ("bf16", 64), ("bf16", 128)])
+@pytest.mark.parametrize("H,Sq,S,splits", [(3, 2, 64, 0), (8, 16, 1000, 0), (3, 17, 4160, 7), (2, 128, 4096, 33),
+                                           (8, 129, 130, 2), (5, 260, 5000, 0)], ids=lambda x: str(x))
+def test_attend_query_blocks(dtype, d, H, Sq, S, splits):
+    """oc_attend at its edges: query counts around a wave's 16 and a block's
+    128, a partial last tile, masks that leave shares (and everything) empty,
+    more mask words than one, 2..33 partials per row (the one-round merge takes
+    at most 32) and one share; K and V are views of a longer cache."""
+    from orthocache_gpu import _launch as X
+    g = torch.Generator().manual_seed(Sq + S)
+    q = torch.randn((Sq, H, d), generator=g).to(TD[dtype]).to(DEV)
+    k, v = (torch.randn((S + 3, H + 1, d), generator=g).to(TD[dtype]).to(DEV)[:S, :H] for _ in range(2))
+    T = -(-S // 64)
+    masks = [None, torch.zeros(T, dtype=torch.uint8), (torch.rand(T, generator=g) < 0.3).to(torch.uint8)]
+    masks[2][T - 1] = 1
+    print(f"attend {dtype} d={d} H={H} Sq={Sq} S={S} splits={splits}", flush=True)
+    for m in masks:
+        out = X.attend(q, k, v, TD[dtype], tile_mask=None if m is None else m.to(DEV), num_splits=splits)
+        keep = np.ones(S, dtype=bool) if m is None else np.repeat(m.numpy().astype(bool), 64)[:S]
+        if not keep.any():
+            assert not out.any()
+            continue
+        logits = np.einsum("qhd,khd->hqk", np64(q), np64(k)[keep]) / np.sqrt(d)
+        p = np.exp(logits - logits.max(axis=2, keepdims=True))
+        ref = np.einsum("hqk,khd->qhd", p / p.sum(axis=2, keepdims=True), np64(v)[keep])
+        assert_out(out, ref, dtype, f"attend {dtype} d={d} Sq={Sq} S={S} masked={m is not None}")
+
+
+@pytest.mark.parametrize("P", [1, 8, 9, 16, 17, 32, 33])
+@pytest.mark.parametrize("d", [4, 64, 96, 256])
+def test_merge_of_few_partials(P, d):
+    """The one-round merge at the ends of its forms (8, 16, 32 partials), and
+    the shapes that keep the general one, with empty partials (m = -inf)."""
+    from orthocache_gpu import _launch as X
+    g = torch.Generator().manual_seed(P * 1000 + d)
+    rows = 37
+    m, l = torch.randn((rows, P), generator=g) * 5, torch.rand((rows, P), generator=g) + 0.5
+    acc = torch.randn((rows, P, d), generator=g)
+    m[::3, 1:] = float("-inf")
+    w = np.exp(np64(m) - np64(m).max(axis=1, keepdims=True))
+    ref = (w[:, :, None] * np64(acc)).sum(axis=1) / (w * np64(l)).sum(axis=1)[:, None]
+    got = X.lse_merge(m.to(DEV), l.to(DEV), acc.to(DEV))
+    # P float32 products per value, weights exp() of differences up to about 40
+    np.testing.assert_allclose(np64(got), ref, atol=1e-5, rtol=1e-5)
