@@ -12,6 +12,7 @@ import threading
 from dataclasses import dataclass
 from typing import Dict, Optional, Tuple
 
+import numpy as np
 import torch
 
 from . import _native as N
@@ -323,7 +324,10 @@ def decode(kv: KVLayout, q: torch.Tensor, G: int, *, gate: int, threshold: float
         raise ValueError(f"out must be a ({rows_q}, {d}) tensor on {device} with a contiguous last dim")
     keep = None
     if want_keep:
-        keep = torch.zeros((kv.num_rows, max(kv.num_tiles, 1)), dtype=torch.uint8, device=device)
+        # every gate writes the flag of every tile of a row; tiles past a
+        # row's length have none and read 0
+        make = torch.zeros if kv.lengths is not None or kv.num_tiles == 0 or gate == N.OC_GATE_NONE else torch.empty
+        keep = make((kv.num_rows, max(kv.num_tiles, 1)), dtype=torch.uint8, device=device)
     p = N.OcDecodeParams()
     p.kv = kv.struct()
     p.q = q.data_ptr()
@@ -684,8 +688,29 @@ def masked_decode(q: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, til
     return out
 
 
-def counts_metadata(keep: torch.Tensor, tiles_total: int) -> dict:
-    retained = int(keep.sum().item())
+_COUNT_HOST = threading.local()
+_COUNT_HOST_BYTES = 1 << 20  # flags beyond this are summed on the GPU
+
+
+def counts_metadata(keep: torch.Tensor, tiles_total) -> dict:
+    """Waits for the device, then the counts of a decode's keep flags (rows,
+    tiles) uint8.  tiles_total: the number of tiles, or a function called
+    after the wait.  The flags travel to pinned host memory (one buffer per
+    thread, read before this returns) ahead of the wait and are counted there:
+    a sum on the GPU would be another launch and a second wait."""
+    n = keep.numel()
+    flags = None
+    if 0 < n <= _COUNT_HOST_BYTES:
+        buf = getattr(_COUNT_HOST, "buf", None)
+        if buf is None or buf.numel() < n:
+            buf = _COUNT_HOST.buf = torch.empty((max(n, 1 << 14),), dtype=torch.uint8, pin_memory=True)
+        flags = buf[:n]
+        with torch.cuda.device(keep.device):
+            flags.view(keep.shape).copy_(keep, non_blocking=True)
+    torch.cuda.synchronize(keep.device)
+    retained = int(np.count_nonzero(flags.numpy())) if flags is not None else int(keep.sum().item())
+    if callable(tiles_total):
+        tiles_total = tiles_total()
     evicted = tiles_total - retained
     return {"tiles_retained": retained, "tiles_evicted": evicted,
             "eviction_rate": evicted / max(1, tiles_total)}

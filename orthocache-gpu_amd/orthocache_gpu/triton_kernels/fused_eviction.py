@@ -111,9 +111,9 @@ def fused_orthocache_attention_v2(
         "tile_assignment": "interleaved",
     }
     if sync:
-        torch.cuda.synchronize(device)
-        metadata.update(X.counts_metadata(res.keep[:, :num_tiles], num_tiles * num_heads))
-        metadata["eviction_mask"] = res.keep[:, :num_tiles].bool()
+        keep = res.keep[:, :num_tiles]
+        metadata.update(X.counts_metadata(keep, num_tiles * num_heads))
+        metadata["eviction_mask"] = keep.view(torch.bool)
     if return_partials:
         metadata["partials"] = res.partials
     return res.out, metadata
@@ -161,8 +161,7 @@ def fused_orthocache_attention(
                    want_keep=sync or return_mask)
     metadata: Dict[str, Any] = {}
     if sync:
-        torch.cuda.synchronize(device)
         metadata.update(X.counts_metadata(res.keep[:, :num_tiles], num_tiles))
     if return_mask:
-        metadata["eviction_mask"] = res.keep[0, :num_tiles].bool()
+        metadata["eviction_mask"] = res.keep[0, :num_tiles].view(torch.bool)
     return res.out, metadata

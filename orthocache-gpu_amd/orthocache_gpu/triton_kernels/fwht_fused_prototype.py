@@ -63,7 +63,7 @@ def triton_fwht_eviction(
     kv = X.rows_layout(keys.unsqueeze(0), None, tile_size=tile_size)
     kv.num_tiles = num_tiles
     _, _, zeta, keep = X.score_tiles(kv, zeta_max, want_zeta=return_zeta, want_keep=True)
-    mask = keep[0, :num_tiles].bool()
+    mask = keep[0, :num_tiles].view(torch.bool)  # the kernel's 0 / 1 bytes
     return mask, (zeta[0, :num_tiles] if return_zeta else None)
 
 
@@ -91,7 +91,7 @@ def score_tiles(keys: torch.Tensor, zeta_max: float = 0.0, k_scale=None, *, tile
             kv.k_scale_mode, kv.k_scale = X.N.OC_KSCALE_NONE, 1.0
     e_low, e_high, zeta, keep = X.score_tiles(kv, zeta_max)
     return TileScores(e_low[:, :kv.num_tiles], e_high[:, :kv.num_tiles], zeta[:, :kv.num_tiles],
-                      keep[:, :kv.num_tiles].bool(), zeta_max=zeta_max, tile_size=tile_size)
+                      keep[:, :kv.num_tiles].view(torch.bool), zeta_max=zeta_max, tile_size=tile_size)
 
 
 class TileScores:

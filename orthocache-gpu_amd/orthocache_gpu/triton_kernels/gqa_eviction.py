@@ -92,13 +92,14 @@ def fused_orthocache_attention_v3_gqa(
         "gate_type": "cauchy_schwarz",
     }
     if sync:
-        torch.cuda.synchronize(device)
-        if context_lens is None:
-            total = num_tiles * num_kv_heads
-        else:
-            total = int(((kv.lengths.clamp(min=0, max=seq_len) + tile_size - 1) // tile_size).sum().item())
-        metadata.update(X.counts_metadata(res.keep[:, :num_tiles], total))
-        metadata["eviction_mask"] = res.keep[:, :num_tiles].bool()
+        def total():
+            if context_lens is None:
+                return num_tiles * num_kv_heads
+            return int(((kv.lengths.clamp(min=0, max=seq_len) + tile_size - 1) // tile_size).sum().item())
+
+        keep = res.keep[:, :num_tiles]
+        metadata.update(X.counts_metadata(keep, total))
+        metadata["eviction_mask"] = keep.view(torch.bool)
     if return_partials:
         metadata["partials"] = res.partials
     return res.out, metadata

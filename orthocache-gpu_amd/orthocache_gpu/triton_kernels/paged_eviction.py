@@ -146,14 +146,14 @@ def fused_orthocache_attention_paged(
         "layout": "paged",
     }
     if sync:
-        torch.cuda.synchronize(device)
-        if int(kv.error_flag.item()) != 0:
-            raise ValueError("block_tables holds a block id outside [0, num_blocks)")
-        if context_lens is None:
-            total = num_tiles * rows
-        else:
+        def total():
+            if int(kv.error_flag.item()) != 0:
+                raise ValueError("block_tables holds a block id outside [0, num_blocks)")
+            if context_lens is None:
+                return num_tiles * rows
             lens = kv.lengths.clamp(min=0, max=num_tiles * tile_size)
-            total = int(((lens + tile_size - 1) // tile_size).sum().item()) * num_kv_heads
+            return int(((lens + tile_size - 1) // tile_size).sum().item()) * num_kv_heads
+
         metadata.update(X.counts_metadata(res.keep[:, :num_tiles], total))
     return res.out.view(num_seqs, num_heads, head_dim), metadata
 
