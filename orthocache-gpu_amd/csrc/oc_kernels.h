@@ -5,7 +5,8 @@
 // Wavefront layout of one 64-token tile (all dtypes, head_dim D = 16*CPL):
 //   lane  = 16*gamma + j            (gamma = 0..3, j = 0..15)
 //   token = 4*i + gamma             (i = 0..15, one "register row" per i)
-//   dims  = CPL*j .. CPL*j + CPL-1  (CPL = D/16 consecutive elements)
+//   dims  = CPL*j .. CPL*j + CPL-1  (CPL = D/16 consecutive elements;
+//           float32 at D = 128: 4j .. 4j+3 and 64+4j .. 64+4j+3)
 // One load instruction of the wave therefore covers 4 whole token rows
 // (64 lanes x CPL elements), so every global load is fully coalesced.
 // Token bits t2..t5 live in the register index i, t0..t1 in the lane bits
@@ -151,6 +152,16 @@ struct Lay {
   static constexpr int LB = CPL * Elem<DT>::size;  // bytes per lane per register row
   static constexpr int LW = LB / 4;                // 32-bit words
   static_assert(LB >= 4 && LB <= 32, "unsupported lane width");
+  // A lane's columns are contiguous up to one 16-byte load.  32 bytes
+  // (float32 at D = 128) are two pieces half a row apart, so that each load
+  // instruction still covers whole 256-byte runs: with adjacent pieces every
+  // instruction touched every second 16 bytes of a row, and each line was
+  // asked for twice (32 float32 heads x 32768 tokens, half retained, single
+  // pass: 146.5 -> 131.6 us; cached 101 -> 91).
+  static constexpr int PIECE = LB < 16 ? LB : 16;       // bytes per load
+  static constexpr int EPP = PIECE / Elem<DT>::size;    // columns per piece
+  // column of the lane's value c (c < CPL)
+  __device__ static constexpr int col(int j, int c) { return 16 * EPP * (c / EPP) + EPP * j + c % EPP; }
 };
 
 // ---------------------------------------------------------------- lane ops
@@ -298,7 +309,7 @@ __device__ __forceinline__ void load_lane_row(const char* p, uint32_t* w) {
   typedef uint32_t v2u __attribute__((ext_vector_type(2)));
   if constexpr (LB == 32) {
     const v4u a = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(p));
-    const v4u b = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(p + 16));
+    const v4u b = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(p + 256));  // Lay::PIECE * 16 lanes on
     w[0] = a[0]; w[1] = a[1]; w[2] = a[2]; w[3] = a[3];
     w[4] = b[0]; w[5] = b[1]; w[6] = b[2]; w[7] = b[3];
   } else if constexpr (LB == 16) {
@@ -412,7 +423,7 @@ template <int LB>
 __device__ __forceinline__ void buffer_load_lane_row(__amdgpu_buffer_rsrc_t r, int voff, int soff, uint32_t* w) {
   if constexpr (LB == 32) {
     const auto x = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, kStreamAux);
-    const auto y = __builtin_amdgcn_raw_buffer_load_b128(r, voff + 16, soff, kStreamAux);
+    const auto y = __builtin_amdgcn_raw_buffer_load_b128(r, voff + 256, soff, kStreamAux);  // Lay::PIECE * 16 lanes on
     w[0] = x[0]; w[1] = x[1]; w[2] = x[2]; w[3] = x[3];
     w[4] = y[0]; w[5] = y[1]; w[6] = y[2]; w[7] = y[3];
   } else if constexpr (LB == 16) {
@@ -447,7 +458,7 @@ __device__ __forceinline__ void load_tile(const DecodeArgs& a, const RowInfo& ri
     const int64_t ts = is_v ? a.v_tok_stride : a.k_tok_stride;
     const char* base = (is_v ? a.v : a.k) + (int64_t)row * (is_v ? a.v_row_stride : a.k_row_stride) + tok0 * ts;
     const int nbytes = (int)(min(valid, 64) * ts);
-    const int voff = gamma * (int)ts + j * L::LB;
+    const int voff = gamma * (int)ts + j * L::PIECE;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       // one descriptor per 4-token row keeps the lane offset in one VGPR; the
@@ -462,7 +473,7 @@ __device__ __forceinline__ void load_tile(const DecodeArgs& a, const RowInfo& ri
     const int64_t bstride = is_v ? a.v_blk_stride : a.k_blk_stride;
     const int64_t hoff = (int64_t)ri.head * (is_v ? a.v_head_stride : a.k_head_stride);
     const int64_t ts = is_v ? a.v_tok_stride : a.k_tok_stride;
-    const int64_t lane_off = (int64_t)j * L::LB;
+    const int64_t lane_off = (int64_t)j * L::PIECE;
     const int32_t* btrow = a.bt + (int64_t)ri.seq * a.bt_stride;
     const int bmask = (1 << a.bs_log2) - 1;
 #pragma unroll
@@ -736,7 +747,7 @@ __device__ __forceinline__ void tile_softmax(WaveState<GT>& st, float (&acc)[GT]
       for (int x = 0; x < QW; ++x) qp[x] = sh_qp[g * (D / 2) + j * QW + x];
     } else {
 #pragma unroll
-      for (int c = 0; c < CPL; ++c) qf[c] = sh_qf[g * D + j * CPL + c];
+      for (int c = 0; c < CPL; ++c) qf[c] = sh_qf[g * D + Lay<DT, D>::col(j, c)];
     }
     // computed in every lane (the transpose-reduce reads all lanes), then masked
     float logit = tile_logit<DT, D, DOT2>(kw, qp, qf, lane) * lscale;
@@ -2146,7 +2157,7 @@ __device__ __forceinline__ void decode_body(const DecodeArgs& a, const RowInfo& 
 #pragma unroll
       for (int c = 0; c < CPL; ++c) {
         const float x = rows4_sum(acc[g][c]);
-        if (lane < 16) sh_acc[wave][g][j * CPL + c] = x;
+        if (lane < 16) sh_acc[wave][g][L::col(j, c)] = x;
       }
     }
     if (lane == 0) {
@@ -3271,7 +3282,7 @@ __global__ __launch_bounds__(kThreads) void fwht_kernel(const DecodeArgs a) {
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
 #pragma unroll
-    for (int c = 0; c < CPL; ++c) out[(int64_t)(4 * i + gamma) * D + j * CPL + c] = f[i][c];
+    for (int c = 0; c < CPL; ++c) out[(int64_t)(4 * i + gamma) * D + L::col(j, c)] = f[i][c];
   }
 }
 
