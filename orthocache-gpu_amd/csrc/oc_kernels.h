@@ -856,9 +856,15 @@ __device__ __forceinline__ f32x4 mfma_qk(const uint32_t (&aq)[4], const uint32_t
 }
 
 // A operand: q of head (lane & 15) from the packed LDS copy (zero past GT).
-// Instruction dc takes head-dim columns 32*dc + 8*kg .. +8 from lane group
-// kg; for fp8 K, whose lanes hold D/4 consecutive columns (kg*D/4 ..),
-// columns kg*D/4 + 8*dc .. +8 (any column order works if q and K agree).
+// Instruction dc takes head-dim columns q_col<F8>(kg, dc) .. + 8 from lane
+// group kg (any column order works if q and K agree): 32 dc + 8 kg for 16-bit
+// K; for fp8 K, whose lanes hold the 16-byte pieces 64 p + 16 kg, the halves of
+// piece dc / 2.
+template <bool F8>
+__device__ __forceinline__ constexpr int q_col(int kg, int dc) {
+  return F8 ? 64 * (dc >> 1) + 16 * kg + 8 * (dc & 1) : 32 * dc + 8 * kg;
+}
+
 template <int DT, int D, int GT>
 __device__ __forceinline__ void load_q_mfma(const uint32_t* sh_qp, int lane, uint32_t (&aq)[D / 32][4]) {
   const int x = lane & 15;
@@ -867,14 +873,14 @@ __device__ __forceinline__ void load_q_mfma(const uint32_t* sh_qp, int lane, uin
   for (int dc = 0; dc < D / 32; ++dc)
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
-      const int pair = DT == OC_FP8_E4M3FN ? kg * (D / 8) + 4 * dc + w : 16 * dc + 4 * kg + w;
+      const int pair = q_col<DT == OC_FP8_E4M3FN>(kg, dc) / 2 + w;
       aq[dc][w] = x < GT ? sh_qp[x * (D / 2) + pair] : 0u;
     }
 }
 
 // B operand (eight 16-bit values) of instruction (tb, dc) from the K
-// registers: kb[tb][dc] for 16-bit K; for fp8 K the lane's bytes 8*dc .. +8
-// of its D/4-byte row piece (words 2dc, 2dc + 1), widened to bf16.
+// registers: kb[tb][dc] for 16-bit K; for fp8 K bytes 8*dc .. +8 of the
+// lane's pieces (words 2dc, 2dc + 1), widened to bf16.
 template <int DT, int D>
 __device__ __forceinline__ void k_operand(const uint32_t (&kb)[4][D / 32][4], int tb, int dc, uint32_t (&b)[4],
                                           bool dq = false, float sc = 1.f) {
@@ -936,8 +942,13 @@ __device__ __forceinline__ const char* page_row(const char* pool, int64_t blk_st
 // place in its page) whose size is the valid part of the block, so tokens
 // at or past n_tok read as zero.
 //
-// fp8 K: lane 16*kg + x reads the D/4 bytes kg*D/4 .. of token 16*tb + x
-// (D/64 128-bit loads per block) into kb[tb][0..D/64).
+// fp8 K: lane 16*kg + x reads the 16-byte pieces 64*p + 16*kg of token 16*tb
+// + x (D/64 128-bit loads per block) into kb[tb][0..D/64), so that a load's
+// four lanes of a token cover 64 bytes without a gap, as in 16 bits.  (With the
+// D/4 consecutive bytes kg*D/4 .. per lane, a load touched 16 bytes of every
+// D/4: 32 rows x 32768 tokens of 256, G = 8, half retained, 116.5 -> 95.0 us
+// single pass and 81.0 -> 66.1 cached; of 128, 131072 tokens, 153.7 -> 150.6
+// single pass on one box.)
 template <int DT, int D, bool PAGED>
 __device__ __forceinline__ void load_k_mfma(const DecodeArgs& a, const RowInfo& ri, int row, int t, int lane,
                                             uint32_t (&kb)[4][D / 32][4], const TilePages& pg) {
@@ -948,7 +959,7 @@ __device__ __forceinline__ void load_k_mfma(const DecodeArgs& a, const RowInfo& 
   const int64_t ts = a.k_tok_stride;
   const char* base = a.k + (int64_t)row * a.k_row_stride + tok0 * ts;
   const int nbytes = (int)(min(ri.n_tok - tok0, 64) * ts);
-  const int voff = x * (int)ts + (F8 ? kg * (D / 4) : 16 * kg);
+  const int voff = x * (int)ts + 16 * kg;
 #pragma unroll
   for (int tb = 0; tb < 4; ++tb) {
     const int rb = 16 * tb * (int)ts;
@@ -962,7 +973,7 @@ __device__ __forceinline__ void load_k_mfma(const DecodeArgs& a, const RowInfo& 
     }
 #pragma unroll
     for (int dc = 0; dc < (F8 ? D / 64 : D / 32); ++dc) {
-      const auto v = __builtin_amdgcn_raw_buffer_load_b128(rs, voff + (F8 ? 16 : 64) * dc, 0, kStreamAux);
+      const auto v = __builtin_amdgcn_raw_buffer_load_b128(rs, voff + 64 * dc, 0, kStreamAux);
       kb[tb][dc][0] = v[0];
       kb[tb][dc][1] = v[1];
       kb[tb][dc][2] = v[2];
@@ -1199,7 +1210,7 @@ __device__ __forceinline__ void unpack16x2(uint32_t u, float& lo, float& hi) {
 // The summation order is not that of tile_energies, so the two can differ
 // in the last bits.
 //
-// fp8 K (a lane holds D/4 columns per token, kb[tb][0..D/64)) with a
+// fp8 K (a lane holds D/4 columns of a token, kb[tb][0..D/64)) with a
 // per-tile scale s: the energies of the stored values times s^2 (the
 // energies of the dequantised tile s*k up to float rounding).
 template <int DT, int D, bool LOW>
@@ -1390,13 +1401,13 @@ __device__ __forceinline__ void load_k_mfma_t(const DecodeArgs& a, const RowInfo
   const char* base = a.k + (int64_t)row * a.k_row_stride + tok0 * ts;
   const int nbytes = (int)(min(ri.n_tok - tok0, 64) * ts);
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, nbytes, 0x00020000);
-  const int cofs = F8 ? kg * (D / 4) : 16 * kg;
+  const int cofs = 16 * kg;
 #pragma unroll
   for (int tb = 0; tb < 4; ++tb) {
     const int voff = kperm(16 * tb + x) * (int)ts + cofs;
 #pragma unroll
     for (int dc = 0; dc < (F8 ? D / 64 : D / 32); ++dc) {
-      const auto v = __builtin_amdgcn_raw_buffer_load_b128(rs, voff + (F8 ? 16 : 64) * dc, 0, kStreamAux);
+      const auto v = __builtin_amdgcn_raw_buffer_load_b128(rs, voff + 64 * dc, 0, kStreamAux);
       kb[tb][dc][0] = v[0];
       kb[tb][dc][1] = v[1];
       kb[tb][dc][2] = v[2];
@@ -1420,7 +1431,7 @@ __device__ __forceinline__ void load_k_mfma_t_paged(const DecodeArgs& a, const R
   const int x = lane & 15;
   const int kg = lane >> 4;
   const int64_t ts = a.k_tok_stride;
-  const int cofs = F8 ? kg * (D / 4) : 16 * kg;
+  const int cofs = 16 * kg;
   const int bmask = (1 << a.bs_log2) - 1;
   const int64_t head_off = (int64_t)ri.head * a.k_head_stride;
 #pragma unroll
@@ -1433,7 +1444,7 @@ __device__ __forceinline__ void load_k_mfma_t_paged(const DecodeArgs& a, const R
     const char* rp = page_row(a.k, a.k_blk_stride, head_off, ts, ok ? id : -1, t * 64 + tok, bmask) + cofs;
 #pragma unroll
     for (int dc = 0; dc < (F8 ? D / 64 : D / 32); ++dc) {
-      const v4u v = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(rp + (F8 ? 16 : 64) * dc));
+      const v4u v = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(rp + 64 * dc));
       kb[tb][dc][0] = ok ? v[0] : 0u;
       kb[tb][dc][1] = ok ? v[1] : 0u;
       kb[tb][dc][2] = ok ? v[2] : 0u;
@@ -2197,14 +2208,14 @@ __device__ __forceinline__ void decode_fast(const DecodeArgs& a, const RowInfo& 
   const bool cached = a.mode == OC_MODE_CACHED && a.gate != OC_GATE_NONE;
 
   // q operand (B of S^T = K.q^T): lane 16 kg + x holds q[head x] columns
-  // 32 dc + 8 kg .. + 8 (fp8 K: kg D / 4 + 8 dc ..), zero past G; one 16-byte
+  // q_col(kg, dc) .. + 8, zero past G; one 16-byte
   // load per instruction column block, straight from q
   uint32_t aq[D / 32][4];
   auto load_q = [&]() {
     const char* qh = a.q + ((int64_t)row * a.G + x) * a.q_row_stride;
 #pragma unroll
     for (int dc = 0; dc < D / 32; ++dc) {
-      const int e0 = F8 ? kg * (D / 4) + 8 * dc : 32 * dc + 8 * kg;
+      const int e0 = q_col<F8>(kg, dc);
       uint4 v = make_uint4(0u, 0u, 0u, 0u);
       if (x < a.G) v = *reinterpret_cast<const uint4*>(qh + 2 * e0);
       aq[dc][0] = v.x;
