@@ -487,3 +487,30 @@ def test_selection_of_clustered_long_and_odd_rows():
         for k in (0, 1, (n - 1) // 2, n - 1):
             sel = X.kth_smallest(x.to(DEV), k).cpu().numpy()
             assert np.array_equal(sel, srt[:, k], equal_nan=True), (n, k)
+
+
+@pytest.mark.parametrize("dtype,d", [("f32", 64), ("f32", 128), ("f16", 128), ("bf16", 64), ("bf16", 128)])
+@pytest.mark.parametrize("scale", [None, 0.05, -0.05, 0.0])
+def test_prefill_tile_words_scales_and_moving_maxima(dtype, d, scale):
+    """The prefill's tile walk over more than one 64-tile word (a whole word
+    evicted, a word with one tile left, the partial last tile), softmax scales
+    of either sign and zero, and keys that grow along the context, so that
+    the running max passes its reference by less and by more than the slack;
+    with the entropy (its sums use the same reference)."""
+    from orthocache_gpu import _launch as X
+    B, Hq, Hkv, Sq, Skv = 1, 4, 2, 150, 64 * 130 + 7
+    q, k, v = _qkv(B, Hq, Hkv, Sq, Skv, d, dtype, seed=61)
+    ramp = torch.linspace(0.05, 3.0, Skv, device=DEV).view(1, 1, -1, 1)
+    k = (k.float() * ramp).to(TD[dtype])
+    T = Skv // 64
+    g = torch.Generator().manual_seed(62)
+    evict = torch.rand((B, Hkv, T), generator=g) < 0.4
+    evict[0, 0, :64] = True           # the first word has no tile left
+    evict[0, 1, 64:128] = True
+    evict[0, 1, 100] = False          # the second has one
+    s = 1.0 / d ** 0.5 if scale is None else scale
+    print(f"prefill words {dtype} d={d} scale={scale}", flush=True)
+    out, ent = X.prefill_attention(q, k, v, tile_mask=evict.to(torch.uint8).to(DEV), scale=scale, want_entropy=True)
+    ref, ref_ent = O.hook_causal_attention(np64(q) * (s * d ** 0.5), np64(k), np64(v), Hq // Hkv, evict.numpy())
+    assert_out(out, ref, dtype, f"prefill words {dtype} d={d} scale={scale}")
+    np.testing.assert_allclose(np64(ent), ref_ent, atol=1e-4, rtol=2e-5)
