@@ -50,6 +50,7 @@ struct PrefillArgs {
   float* entropy;  // (B, Hq, Sq) or null
   int32_t qblocks;
   int32_t o_vec;  // out rows 8-byte aligned
+  int32_t rev;    // query blocks dispatched longest first; those after them shortest first
   // split windows (nitems > 0): work item e is query block items[e] >> 2,
   // part items[e] & 3 (0: its whole window; 1, 2: the first and second half
   // of its tiles).  Blocks >= q0 are split: (block, head) pair k of them keeps
@@ -485,7 +486,9 @@ __global__ __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(DT =
     bh = i % nbh;
     e = i / nbh;
   }
-  int qb = a.qblocks - 1 - e, part = 0;
+  // (a call of at most two workgroups per CU: the second ones, e >= a.rev,
+  // shortest first)
+  int qb = e < a.rev ? a.qblocks - 1 - e : e - a.rev, part = 0;
   if constexpr (SPLIT) {
     qb = a.items[e] >> 2;
     part = a.items[e] & 3;
@@ -1443,12 +1446,33 @@ int pf_slots_t() {
   return per_cu[dev] > 0 ? per_cu[dev] * cus[dev] : 0;
 }
 
+int pf_cus() {
+  int dev = 0, c = 0;
+  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return 0;
+  return c;
+}
+
 int pf_slots(int dtype, int d) {
   switch (dtype) {
     case OC_F32: return d == 64 ? pf_slots_t<OC_F32, 64>() : pf_slots_t<OC_F32, 128>();
     case OC_F16: return d == 64 ? pf_slots_t<OC_F16, 64>() : pf_slots_t<OC_F16, 128>();
     default: return d == 64 ? pf_slots_t<OC_BF16, 64>() : pf_slots_t<OC_BF16, 128>();
   }
+}
+
+// When a call's workgroups all fit the device at once, at most two to a CU,
+// the first n of a head's `items` work items (longest first) go one to each CU
+// and the rest join them: shortest first, so that every CU gets about the same
+// sum of windows.  (Longest first throughout gave the CUs with the longest
+// window the longest of the rest: 32 float32 heads x 1999 x 64, none / a quarter
+// / half of the tiles evicted, 195 / 159 / 118 us against 152 / 126 / 94; 2048 x
+// 64 in bfloat16 50.5 / 43.5 / 31.7 against 49.3 / 38.3 / 31.2.)
+int pf_first_fill(const oc_prefill_params* p, int items) {
+  const int64_t nbh = (int64_t)p->batch * p->num_q_heads;
+  const int slots = pf_slots(p->dtype, p->head_dim), cus = pf_cus();
+  if (cus <= 0 || slots < 2 * cus || nbh * items > 2 * (int64_t)cus || nbh > cus) return items;
+  return (int)std::min<int64_t>(items, cus / nbh);
 }
 
 constexpr size_t kPfCounterBytes = 64 << 10;
@@ -1475,6 +1499,16 @@ bool pf_plan(const oc_prefill_params* p, PfPlan* pl) {
   if (qblocks < 1 || nbh < 1) return false;
   const int slots = pf_slots(p->dtype, p->head_dim);
   if (slots <= 0 || nbh * qblocks > slots) return false;
+  // At head_dim 128, a call that nearly fills two workgroups to a CU with at
+  // most 16 or so blocks a head is better off with the paired windows of
+  // pf_first_fill than with a split whose halves no longer fit at once (32 heads
+  // x 2043, split against paired: float16 59.8 / 52.1 us, bfloat16 66.9 / 63.2;
+  // x 1531 35.2 / 37.3 and 42.0 / 45.3; 16 heads x 3579 in bfloat16 97 / 101).
+  // head_dim 64 keeps the split (32 x 2043: float32 156 / 155, bfloat16 47.1 /
+  // 47.7; 8 heads x 8187: 576 / 589 and 150 / 177).
+  const int64_t cus = pf_cus();
+  if (p->head_dim == 128 && nbh * 8 >= cus && nbh * qblocks * 8 >= 14 * cus && pf_first_fill(p, qblocks) < qblocks)
+    return false;
   const int off = p->kv_len - p->q_len;
   auto window = [&](int qb) {
     return (std::min(std::max(std::min(qb * kPfRows + kPfRows - 1, p->q_len - 1) + off + 1, 0), p->kv_len) + 63) / 64;
@@ -1565,6 +1599,7 @@ extern "C" int oc_prefill_attention(const oc_prefill_params* p, void* stream) {
   a.qblocks = (p->q_len + kPfRows - 1) / kPfRows;
   a.o_vec = ((uintptr_t)p->out | (uintptr_t)a.o_sb | (uintptr_t)a.o_sh | (uintptr_t)a.o_ss) % 8 == 0;
   int64_t items = a.qblocks;
+  a.rev = pf_first_fill(p, a.qblocks);
   if (p->workspace) {
     PfPlan pl;
     if (pf_plan(p, &pl)) {

@@ -514,3 +514,33 @@ def test_prefill_tile_words_scales_and_moving_maxima(dtype, d, scale):
     ref, ref_ent = O.hook_causal_attention(np64(q) * (s * d ** 0.5), np64(k), np64(v), Hq // Hkv, evict.numpy())
     assert_out(out, ref, dtype, f"prefill words {dtype} d={d} scale={scale}")
     np.testing.assert_allclose(np64(ent), ref_ent, atol=1e-4, rtol=2e-5)
+
+
+@pytest.mark.parametrize("dtype,d", [("f32", 64), ("f16", 64), ("bf16", 128), ("f16", 128)])
+@pytest.mark.parametrize("S", [600, 1000])  # 64 heads: 5 and 8 query blocks, one CU's share is 4
+@pytest.mark.parametrize("masked", [False, True], ids=["plain", "masked"])
+def test_prefill_paired_windows_vs_oracle(dtype, d, S, masked):
+    """Calls of one to two workgroups per CU, whose second ones run shortest
+    window first; unmasked they are split unless head_dim 128 nearly fills both."""
+    import ctypes
+    from orthocache_gpu import _launch as X
+    from orthocache_gpu import _native as N
+    B, Hq, Hkv = 2, 32, 4
+    q, k, v = _qkv(B, Hq, Hkv, S, S, d, dtype, seed=S + d)
+    evict, tm = None, None
+    if masked:
+        evict = torch.rand((B, Hkv, S // 64), generator=torch.Generator().manual_seed(S)) < 0.4
+        tm = evict.to(torch.uint8).to(DEV)
+    p = N.OcPrefillParams()
+    p.dtype, p.batch, p.num_q_heads, p.num_kv_heads = X.dtype_code(q.dtype, "q"), B, Hq, Hkv
+    p.q_len, p.kv_len, p.head_dim = S, S, d
+    if masked:
+        p.tile_mask, p.tile_mask_cols = tm.data_ptr(), S // 64
+    elif torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert (N.lib().oc_prefill_workspace_size(ctypes.byref(p)) > 0) == (not (d == 128 and S == 1000))
+    print(f"prefill paired {dtype} d={d} S={S} masked={masked}", flush=True)
+    out, ent = X.prefill_attention(q, k, v, tile_mask=tm, want_entropy=True)
+    ref, ref_ent = O.hook_causal_attention(np64(q), np64(k), np64(v), Hq // Hkv,
+                                           None if evict is None else evict.numpy())
+    assert_out(out, ref, dtype, f"prefill paired {dtype} d={d} S={S} masked={masked}")
+    np.testing.assert_allclose(np64(ent), ref_ent, atol=1e-4, rtol=1e-5)
