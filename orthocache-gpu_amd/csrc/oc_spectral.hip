@@ -10,9 +10,11 @@
 //   sum_ul ||X[64 uh + ul]||^2 = ||Z_uh||_F^2 / 8.
 // So the bands [64, 256) (uh = 1..3) and [256, 512) (uh = 4..7) are sums of
 // squares of the 8-point outputs, computed in registers as the block
-// streams in; the band [1, 64) and the DC row need the 64-point transform
-// of Z_0 along tl, done per column from LDS.  Every band energy is a sum of
-// squares, so near-zero bands stay exact-ish instead of cancelling.
+// streams in; the band [1, 64) is, by Parseval over tl, what is left of
+// Z_0 without its mean, 64 sum_tl (Z_0[tl] - mean)^2, from the registers too
+// (the generic head_dim path does the 64-point transform per column from
+// LDS).  Every band energy is a sum of squares, so near-zero bands stay
+// exact-ish instead of cancelling.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -48,40 +50,67 @@ struct SpecArgs {
 };
 
 // 16-byte pieces of one token position: the eight chunk values (th) of a
-// thread's eight columns, fetched raw so that no use of the loaded words
-// (no wait) sits among the loads
+// thread's columns (eight 16-bit or four float32), fetched raw so that no use
+// of the loaded words (no wait) sits among the loads
 template <int DT>
 struct SpRaw {
-  static constexpr int N = DT == OC_F32 ? 16 : 8;
-  uint4 w[N];
+  static constexpr int COLS = DT == OC_F32 ? 4 : 8;
+  u32x4 w[8];
 };
 
+// K streams past the caches (32 heads x 32K x 128 in bfloat16 52.9 us with
+// plain loads, 48.5 streamed; x 16K in float32 48.2 / 42.1).  The compact
+// pipeline's decode, which reads the retained half again, then takes 54 us
+// where it took 49, so the two together are level; callers of the spectra
+// alone keep the gain.
 template <int DT>
 __device__ __forceinline__ void sp_fetch(const char* p, int64_t th_stride, SpRaw<DT>& r) {
 #pragma unroll
-  for (int th = 0; th < 8; ++th) {
-    const char* pt = p + th * th_stride;
-    if constexpr (DT == OC_F32) {
-      r.w[2 * th] = *reinterpret_cast<const uint4*>(pt);
-      r.w[2 * th + 1] = *reinterpret_cast<const uint4*>(pt + 16);
-    } else {
-      r.w[th] = *reinterpret_cast<const uint4*>(pt);
-    }
-  }
+  for (int th = 0; th < 8; ++th)
+    r.w[th] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p + th * th_stride));
 }
 
 // column c of chunk th as float
 template <int DT>
 __device__ __forceinline__ float sp_elem(const SpRaw<DT>& r, int th, int c) {
   if constexpr (DT == OC_F32) {
-    const uint4 u = r.w[2 * th + c / 4];
-    const uint32_t x = (c & 3) == 0 ? u.x : (c & 3) == 1 ? u.y : (c & 3) == 2 ? u.z : u.w;
-    return __uint_as_float(x);
+    return __uint_as_float(r.w[th][c]);
   } else {
-    const uint4 u = r.w[th];
-    const uint32_t x = (c >> 1) == 0 ? u.x : (c >> 1) == 1 ? u.y : (c >> 1) == 2 ? u.z : u.w;
+    const uint32_t x = r.w[th][c >> 1];
     if constexpr (DT == OC_BF16) return __uint_as_float((c & 1) ? (x & 0xFFFF0000u) : (x << 16));
     else return (float)__builtin_bit_cast(_Float16, (uint16_t)((c & 1) ? (x >> 16) : (x & 0xFFFFu)));
+  }
+}
+
+// Energies of one token position's columns and the 8-point transform over the
+// chunks th; z0[c] receives Z_0.
+template <int DT>
+__device__ __forceinline__ void sp_consume(const SpRaw<DT>& r, float& energy, float& e_mid, float& e_high,
+                                           float (&z0)[SpRaw<DT>::COLS]) {
+#pragma unroll
+  for (int c = 0; c < SpRaw<DT>::COLS; ++c) {
+    float z[8];
+#pragma unroll
+    for (int th = 0; th < 8; ++th) {
+      z[th] = sp_elem<DT>(r, th, c);
+      energy = __builtin_fmaf(z[th], z[th], energy);
+    }
+    // natural-order 8-point Walsh-Hadamard transform over th (unnormalised)
+#pragma unroll
+    for (int m = 1; m < 8; m <<= 1)
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (!(i & m)) {
+          const float u = z[i], v = z[i + m];
+          z[i] = u + v;
+          z[i + m] = u - v;
+        }
+#pragma unroll
+    for (int uh = 1; uh < 4; ++uh) e_mid = __builtin_fmaf(z[uh], z[uh], e_mid);
+#pragma unroll
+    for (int uh = 4; uh < 8; ++uh) e_high = __builtin_fmaf(z[uh], z[uh], e_high);
+    z0[c] = z[0];
+    asm volatile("" : "+v"(z0[c]), "+v"(energy), "+v"(e_mid), "+v"(e_high));  // column by column: few live registers
   }
 }
 
@@ -103,28 +132,225 @@ __device__ __forceinline__ float sp_q_value(uint32_t bits, int dtype) {
   return (float)__builtin_bit_cast(_Float16, (uint16_t)bits);
 }
 
+// The band energies of one (block, head) from its four sums, written by one thread.
+__device__ __forceinline__ float sp_write(const SpecArgs& a, int64_t o, float mid, float high, float low, float energy,
+                                          bool write) {
+  const float s_mid = mid * 0.125f;
+  const float s_high = high * 0.125f;
+  const float s_ac = low + s_mid + s_high;
+  if (write) {
+    if (a.e_low) a.e_low[o] = low;
+    if (a.e_mid) a.e_mid[o] = s_mid;
+    if (a.e_high) a.e_high[o] = s_high;
+    if (a.zeta) a.zeta[o] = s_high / (low + 1e-6f);
+    if (a.e_ac) a.e_ac[o] = s_ac;
+    if (a.energy) a.energy[o] = energy;
+  }
+  return s_ac;
+}
+
+// Eight consecutive elements of a q row, raw: 16-byte loads where every row
+// allows them, else element by element.
+__device__ __forceinline__ void sp_q8(const char* p, int dtype, bool vec, u32x4 (&r)[2]) {
+  if (vec) {
+    r[0] = *reinterpret_cast<const u32x4*>(p);
+    if (dtype == OC_F32) r[1] = *reinterpret_cast<const u32x4*>(p + 16);
+  } else if (dtype == OC_F32) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r[i >> 2][i & 3] = reinterpret_cast<const uint32_t*>(p)[i];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint16_t* e = reinterpret_cast<const uint16_t*>(p) + 2 * i;
+      r[0][i] = (uint32_t)e[0] | ((uint32_t)e[1] << 16);
+    }
+  }
+}
+
+// element c of them as float
+__device__ __forceinline__ float sp_q8_value(const u32x4 (&r)[2], int dtype, int c) {
+  if (dtype == OC_F32) return __uint_as_float(r[c >> 2][c & 3]);
+  const uint32_t x = r[0][c >> 1];
+  return sp_q_value((c & 1) ? (x >> 16) : (x & 0xFFFFu), dtype);
+}
+
+// head_dim 64 and 128: one workgroup per (head, block), HBM-bound.  A thread
+// keeps its positions' Z_0 in registers, so the workgroup needs no Z_0 in LDS
+// and stays below 128 registers a thread (16 wavefronts per CU).  With Z_0 in
+// LDS and the 64-point transform done by half the threads, at 12 wavefronts,
+// 32 heads x 32K x 128 took 53.3 us in bfloat16 and x 16K in float32 52.7, now
+// 48.5 (5.5 TB/s) and 42.1 (6.4 TB/s).  Resident workgroups that walk over the
+// blocks, the next one's loads in flight over the reductions, were slower
+// (58-61 us).
 template <int DT, int D>
-__global__ __launch_bounds__(kSpThreads) void block_spectrum_kernel(const SpecArgs a) {
-  constexpr int DMAX = D ? D : kMaxD;
+__global__ __launch_bounds__(kSpThreads, 4) void block_spectrum_kernel(const SpecArgs a) {
+  constexpr int COLS = SpRaw<DT>::COLS;
+  constexpr int CG = D / COLS;          // threads side by side over a token row (whole rows per instruction)
+  constexpr int TG = kSpThreads / CG;   // token positions at once
+  constexpr int TPT = 64 / TG;          // positions per thread
+  constexpr int WAVES = kSpThreads / 64;
+  static_assert(CG >= 8 && CG <= 32 && TPT >= 2, "lane layout of the column sums");
+  __shared__ float sh_col[WAVES][D];  // column sums of Z_0 per wave
+  __shared__ float sh_mean[D];
+  __shared__ float sh_sum[WAVES][4];
+  __shared__ float sh_red[WAVES];
+  const int tid = threadIdx.x;
+  const int cg = tid % CG;
+  const int tg = tid / CG;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  // consecutive workgroups take the heads of one block, so the workgroups
+  // in flight together read whole token rows of the (S, H, d) cache
+  const int h = blockIdx.x;
+  const int blk = blockIdx.y;
+  const char* kb = a.k + (int64_t)blk * kBlock * a.k_ts + (int64_t)h * a.k_hs + (int64_t)cg * 16 + (int64_t)tg * a.k_ts;
+  // the bounds: D / 8 lanes per query, eight columns each; the wave's first
+  // queries are requested before the block streams in
+  constexpr int LPQ = D / 8, QPW = 64 / LPQ;
+  const int qc = (lane % LPQ) * 8;
+  const int qs = wave * QPW + lane / LPQ;
+  const int qes = a.q_dtype == OC_F32 ? 4 : 2;
+  const bool q_vec = (((uintptr_t)a.q | (uintptr_t)a.q_ss | (uintptr_t)a.q_hs) & 15) == 0;
+  u32x4 q0[2] = {u32x4{0u, 0u, 0u, 0u}, u32x4{0u, 0u, 0u, 0u}};
+  const char* qbase = a.q + (int64_t)h * a.q_hs + (int64_t)qc * qes;
+  if (a.q && qs < a.Sq) sp_q8(qbase + (int64_t)qs * a.q_ss, a.q_dtype, q_vec, q0);
+  const int64_t th_stride = 64 * a.k_ts;
+  SpRaw<DT> rb[2];
+  sp_fetch<DT>(kb, th_stride, rb[0]);
+  // the next position's loads are issued before the current one is consumed
+  float e_mid = 0.f, e_high = 0.f, energy = 0.f;
+  float z0[TPT][COLS];
+#pragma unroll
+  for (int i = 0; i < TPT; ++i) {
+    if (i + 1 < TPT) sp_fetch<DT>(kb + (int64_t)((i + 1) * TG) * a.k_ts, th_stride, rb[(i + 1) & 1]);
+    sp_consume<DT>(rb[i & 1], energy, e_mid, e_high, z0[i]);
+    // the next position but one is not requested before this one is finished
+    // (else the compiler requests every position at once and spills)
+    asm volatile("" : : : "memory");
+  }
+  // column sums over tl, in pairs throughout (a constant column's mean, and
+  // with it E_low = 0, is then exact): the thread's positions, the wave's
+  // lanes of the same columns, the waves
+#pragma unroll
+  for (int c = 0; c < COLS; ++c) {
+    float t[TPT];
+#pragma unroll
+    for (int i = 0; i < TPT; ++i) t[i] = z0[i][c];
+#pragma unroll
+    for (int m = 1; m < TPT; m <<= 1)
+#pragma unroll
+      for (int i = 0; i < TPT; ++i)
+        if (!(i & (2 * m - 1))) t[i] += t[i + m];
+    float x = t[0], lo, hi;
+    if constexpr (CG == 8) x += dpp<0x128>(x);  // row_ror:8
+    if constexpr (CG <= 16) {
+      row_pair<16>(x, lo, hi);
+      x = lo + hi;
+    }
+    row_pair<32>(x, lo, hi);
+    x = lo + hi;
+    if (lane < CG) sh_col[wave][lane * COLS + c] = x;
+  }
+  __syncthreads();
+  auto col_sum = [&](int c) { return (sh_col[0][c] + sh_col[1][c]) + (sh_col[2][c] + sh_col[3][c]); };
+  if (tid < D) {
+    const float m = col_sum(tid) * (1.0f / 512.0f);  // DC / sqrt(512) with DC = sum_t k_t / sqrt(512)
+    sh_mean[tid] = m;
+    if (a.mean) a.mean[((int64_t)blk * a.H + h) * D + tid] = m;
+  }
+  float e_low = 0.f;
+#pragma unroll
+  for (int c = 0; c < COLS; ++c) {
+    const float m = col_sum(cg * COLS + c) * (1.0f / 64.0f);
+#pragma unroll
+    for (int i = 0; i < TPT; ++i) {
+      const float x = z0[i][c] - m;
+      e_low = __builtin_fmaf(x, x, e_low);
+    }
+  }
+  // the four band sums in one reduction: lanes, then the four waves in LDS
+  float r4[4] = {e_mid, e_high, e_low, energy};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) r4[j] = wave_sum(r4[j]);
+  if (lane == 0) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sh_sum[wave][j] = r4[j];
+  }
+  __syncthreads();  // also: sh_mean complete
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    r4[j] = sh_sum[0][j];
+    for (int w = 1; w < WAVES; ++w) r4[j] += sh_sum[w][j];
+  }
+  const int64_t o = (int64_t)blk * a.H + h;
+  const float s_ac = sp_write(a, o, r4[0], r4[1], r4[2] * 0.125f, r4[3], tid == 0);  // 64 / 512
+  if (!a.q) return;
+  // query-aware bounds: (q . mean + ||q|| sqrt(E_ac)) / sqrt(d)
+  const float inv_sd = 1.0f / __builtin_sqrtf((float)D);
+  const float sq_ac = __builtin_sqrtf(fmaxf(s_ac, 0.f));
+  float mean[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) mean[c] = sh_mean[qc + c];
+  float best = -__builtin_inff();
+  float qbest = 0.f;
+  for (int s = qs; s < a.Sq; s += WAVES * QPW) {
+    if (s != qs) sp_q8(qbase + (int64_t)s * a.q_ss, a.q_dtype, q_vec, q0);
+    float dot = 0.f, nn = 0.f;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const float qv = sp_q8_value(q0, a.q_dtype, c);
+      dot = __builtin_fmaf(qv, mean[c], dot);
+      nn = __builtin_fmaf(qv, qv, nn);
+    }
+    // (the lanes of one query leave the loop together)
+    if constexpr (LPQ == 16) {
+      dot += xpair<8>(dot);
+      nn += xpair<8>(nn);
+    }
+    dot += xpair<4>(dot);
+    nn += xpair<4>(nn);
+    dot += xpair<2>(dot);
+    nn += xpair<2>(nn);
+    dot += xpair<1>(dot);
+    nn += xpair<1>(nn);
+    const float qn = __builtin_sqrtf(nn);
+    const float bnd = dot * inv_sd + qn * sq_ac * inv_sd;
+    if (a.bounds && qc == 0) a.bounds[((int64_t)s * a.nb + blk) * a.H + h] = bnd;
+    best = fmaxf(best, bnd);
+    qbest = fmaxf(qbest, qn);
+  }
+  best = block_max(best, sh_red);
+  if (tid == 0 && a.max_bound) a.max_bound[o] = best;
+  if (blk == 0 && a.q_norm_max) {
+    qbest = block_max(qbest, sh_red);
+    if (tid == 0) a.q_norm_max[h] = qbest;
+  }
+}
+
+// Any other head_dim (a multiple of 8 up to kMaxD).
+template <int DT>
+__global__ __launch_bounds__(kSpThreads) void block_spectrum_any_kernel(const SpecArgs a) {
+  constexpr int DMAX = kMaxD;
+  constexpr int COLS = SpRaw<DT>::COLS;
   // Z_0[tl][c]; once the transform has read it (after the barrier that
   // follows), row 0 holds the block mean (each thread writes its own
   // column) and entries d .. d + 20 the reduction scratch, so the whole
   // workgroup's LDS is 32 KiB at d = 128 (five workgroups per CU)
   __shared__ float sh_z[64 * DMAX];
   float* sh_mean = sh_z;
-  float (*sh_sum)[4] = reinterpret_cast<float (*)[4]>(sh_z + (D ? D : a.d));
-  float* sh_red = sh_z + (D ? D : a.d) + 4 * (kSpThreads / 64);
+  float (*sh_sum)[4] = reinterpret_cast<float (*)[4]>(sh_z + a.d);
+  float* sh_red = sh_z + a.d + 4 * (kSpThreads / 64);
   // consecutive workgroups take the heads of one block, so the workgroups
   // in flight together read whole token rows of the (S, H, d) cache
   const int h = blockIdx.x;
   const int blk = blockIdx.y;
-  const int d = D ? D : a.d;
-  const int CG = d / 8;
+  const int d = a.d;
+  const int CG = d / COLS;
   const int TG = kSpThreads / CG;
   const int tid = threadIdx.x;
   const int cg = tid % CG;
   const int tg = tid / CG;
-  const char* kb = a.k + (int64_t)blk * kBlock * a.k_ts + (int64_t)h * a.k_hs + (int64_t)cg * 8 * (DT == OC_F32 ? 4 : 2);
+  const char* kb = a.k + (int64_t)blk * kBlock * a.k_ts + (int64_t)h * a.k_hs + (int64_t)cg * 16;
   // the bounds: wave w takes queries w, w + 4, ..., lane l columns l, l + 64, ...;
   // the wave's first query is requested before the block streams in
   constexpr int QPL = (DMAX + 63) / 64;
@@ -149,58 +375,22 @@ __global__ __launch_bounds__(kSpThreads) void block_spectrum_kernel(const SpecAr
   for (int k = 0; k < QPL; ++k) q0[k] = 0u;
   if (a.q && wave < a.Sq) load_q(wave, q0);
   float e_mid = 0.f, e_high = 0.f, energy = 0.f;
-  // one token position tl of the thread: energies, the 8-point transform
-  // over the chunks th, Z_0 to LDS
-  auto consume = [&](int tl, const SpRaw<DT>& r) {
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      float z[8];
-#pragma unroll
-      for (int th = 0; th < 8; ++th) {
-        z[th] = sp_elem<DT>(r, th, c);
-        energy = __builtin_fmaf(z[th], z[th], energy);
-      }
-      // natural-order 8-point Walsh-Hadamard transform over th (unnormalised)
-#pragma unroll
-      for (int m = 1; m < 8; m <<= 1)
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          if (!(i & m)) {
-            const float u = z[i], v = z[i + m];
-            z[i] = u + v;
-            z[i + m] = u - v;
-          }
-#pragma unroll
-      for (int uh = 1; uh < 4; ++uh) e_mid = __builtin_fmaf(z[uh], z[uh], e_mid);
-#pragma unroll
-      for (int uh = 4; uh < 8; ++uh) e_high = __builtin_fmaf(z[uh], z[uh], e_high);
-      sh_z[tl * d + 8 * cg + c] = z[0];
-    }
-  };
   const int64_t th_stride = 64 * a.k_ts;
-  if constexpr (D != 0) {
-    // TG divides 64: 64 / TG positions per thread, the next position's
-    // loads issued before the current one is consumed
-    constexpr int TPT = 64 / (kSpThreads / (D / 8));
-    SpRaw<DT> rb[2];
-    sp_fetch<DT>(kb + (int64_t)tg * a.k_ts, th_stride, rb[0]);
-#pragma unroll
-    for (int i = 0; i < TPT; ++i) {
-      if (i + 1 < TPT) sp_fetch<DT>(kb + (int64_t)(tg + (i + 1) * TG) * a.k_ts, th_stride, rb[(i + 1) & 1]);
-      consume(tg + i * TG, rb[i & 1]);
-    }
-  } else if (tg < TG) {
-    // any other head_dim: positions tg, tg + TG, ... < 64; the threads past
-    // TG * CG (when CG does not divide 256) take none
+  if (tg < TG) {
+    // positions tg, tg + TG, ... < 64; the threads past TG * CG (when CG does
+    // not divide 256) take none
     for (int tl = tg; tl < 64; tl += TG) {
       SpRaw<DT> r;
+      float z0[COLS];
       sp_fetch<DT>(kb + (int64_t)tl * a.k_ts, th_stride, r);
-      consume(tl, r);
+      sp_consume<DT>(r, energy, e_mid, e_high, z0);
+#pragma unroll
+      for (int c = 0; c < COLS; ++c) sh_z[tl * d + COLS * cg + c] = z0[c];
     }
   }
   __syncthreads();
   // 64-point transform of Z_0 along tl, one column per thread
-  float e_low = 0.f, dc2 = 0.f;
+  float e_low = 0.f;
   if (tid < d) {
     float y[64];
 #pragma unroll
@@ -216,7 +406,6 @@ __global__ __launch_bounds__(kSpThreads) void block_spectrum_kernel(const SpecAr
         }
 #pragma unroll
     for (int i = 1; i < 64; ++i) e_low = __builtin_fmaf(y[i], y[i], e_low);
-    dc2 = y[0] * y[0];
     sh_mean[tid] = y[0] * (1.0f / 512.0f);  // DC / sqrt(512) with DC = sum_t k_t / sqrt(512)
   }
   // the four band sums in one reduction: lanes, then the four waves in LDS
@@ -234,21 +423,8 @@ __global__ __launch_bounds__(kSpThreads) void block_spectrum_kernel(const SpecAr
     r4[j] = sh_sum[0][j];
     for (int w = 1; w < kSpThreads / 64; ++w) r4[j] += sh_sum[w][j];
   }
-  const float s_mid = r4[0] * 0.125f;
-  const float s_high = r4[1] * 0.125f;
-  const float s_low = r4[2] * (1.0f / 512.0f);
-  const float s_energy = r4[3];
-  (void)dc2;
-  const float s_ac = s_low + s_mid + s_high;
   const int64_t o = (int64_t)blk * a.H + h;
-  if (tid == 0) {
-    if (a.e_low) a.e_low[o] = s_low;
-    if (a.e_mid) a.e_mid[o] = s_mid;
-    if (a.e_high) a.e_high[o] = s_high;
-    if (a.zeta) a.zeta[o] = s_high / (s_low + 1e-6f);
-    if (a.e_ac) a.e_ac[o] = s_ac;
-    if (a.energy) a.energy[o] = s_energy;
-  }
+  const float s_ac = sp_write(a, o, r4[0], r4[1], r4[2] * (1.0f / 512.0f), r4[3], tid == 0);
   if (a.mean && tid < d) a.mean[o * d + tid] = sh_mean[tid];
   if (!a.q) return;
   // query-aware bounds: (q . mean + ||q|| sqrt(E_ac)) / sqrt(d)
@@ -310,10 +486,19 @@ __device__ __forceinline__ void gate_reduce(float (&v)[N], unsigned max_mask, fl
     for (int j = 0; j < N; ++j) sh[wave][j] = v[j];
   }
   __syncthreads();
+  // every wave combines the 16 results over the lanes of its rows (read one
+  // by one by all 1024 threads, the LDS reads were most of the reduction)
 #pragma unroll
   for (int j = 0; j < N; ++j) {
-    float t = sh[0][j];
-    for (int w = 1; w < kGateWaves; ++w) t = ((max_mask >> j) & 1) ? fmaxf(t, sh[w][j]) : t + sh[w][j];
+    float t = sh[lane & (kGateWaves - 1)][j];
+    if ((max_mask >> j) & 1) {
+      t = fmaxf(t, xpair<8>(t));
+      t = fmaxf(t, xpair<4>(t));
+      t = fmaxf(t, xpair<2>(t));
+      t = fmaxf(t, xpair<1>(t));
+    } else {
+      t = row16_sum(t);
+    }
     v[j] = t;
   }
 }
@@ -325,25 +510,30 @@ __device__ __forceinline__ void gate_reduce(float (&v)[N], unsigned max_mask, fl
 // retained count, the largest retained bound and the perfect / statistical
 // regimes of the evicted blocks.  stats: [tau, zeta mean, zeta std, zeta
 // min, zeta max, retained, perfect, statistical, z_max].
+//
+// STAGED: at most kGateLds entries and kGateHeads heads, and the tables are
+// read from LDS.  Latency-bound: the masks are stored once per-block results
+// are in LDS, for a wait for any of the loop's reads is one for its earlier
+// stores too (64 blocks of 32 heads: 9.8 us with the stores in the loop and
+// reads that may go to either memory, 6.0 now).
+template <bool STAGED>
 __global__ __launch_bounds__(1024) void compact_gate_kernel(const float* mb, const float* zeta, const float* energy,
                                                             const float* qmax, int nb, int H, int d, float tau_in,
                                                             int tau_auto, float zeta_max, float underflow,
                                                             int tiles_per_block, uint8_t* unified,
                                                             uint8_t* tile_mask, float* stats) {
   __shared__ float sh_f[kGateWaves][8];
-  // the (block, head) tables and the query norms staged in LDS when they
-  // fit, every load in flight at once; otherwise read from global memory
-  __shared__ float sh_mb[kGateLds], sh_zeta[kGateLds], sh_en[kGateLds], sh_qmax[kGateHeads];
+  // the (block, head) tables and the query norms, every load in flight at once
+  __shared__ float sh_mb[STAGED ? kGateLds : 1], sh_zeta[STAGED ? kGateLds : 1], sh_en[STAGED ? kGateLds : 1],
+      sh_qmax[STAGED ? kGateHeads : 1];
   // per-block results of the first pass (any head kept, head-mean zeta, beta)
   __shared__ float sh_za[kGateBlocks], sh_beta[kGateBlocks];
   __shared__ uint8_t sh_any[kGateBlocks];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
   const int n = nb * H;
-  const bool staged = n <= kGateLds && H <= kGateHeads;
-  const bool cache_blk = nb <= kGateBlocks;
-  if (staged) {
+  const bool cache_blk = STAGED || nb <= kGateBlocks;
+  if constexpr (STAGED) {
 #pragma unroll
     for (int k = 0; k < kGateLds / 1024; ++k) {
       const int i = tid + 1024 * k;
@@ -355,25 +545,35 @@ __global__ __launch_bounds__(1024) void compact_gate_kernel(const float* mb, con
     }
     if (tid < H) sh_qmax[tid] = qmax[tid];
     __syncthreads();
-    mb = sh_mb;
-    zeta = sh_zeta;
-    energy = sh_en;
-    qmax = sh_qmax;
   }
+  auto mb_at = [&](int64_t i) { return STAGED ? sh_mb[STAGED ? i : 0] : mb[i]; };
+  auto zeta_at = [&](int64_t i) { return STAGED ? sh_zeta[STAGED ? i : 0] : zeta[i]; };
+  auto energy_at = [&](int64_t i) { return STAGED ? sh_en[STAGED ? i : 0] : energy[i]; };
+  auto qmax_at = [&](int64_t i) { return STAGED ? sh_qmax[STAGED ? i : 0] : qmax[i]; };
   float tau = tau_in;
   if (tau_auto) {
     float s[1] = {0.f};
-    for (int i = tid; i < n; i += 1024) s[0] += mb[i];
+    for (int i = tid; i < n; i += 1024) s[0] += mb_at(i);
     gate_reduce<1>(s, 0u, sh_f);
     const float mean = s[0] / (float)n;
     float v[1] = {0.f};
-    for (int i = tid; i < n; i += 1024) v[0] = __builtin_fmaf(mb[i] - mean, mb[i] - mean, v[0]);
+    for (int i = tid; i < n; i += 1024) v[0] = __builtin_fmaf(mb_at(i) - mean, mb_at(i) - mean, v[0]);
     gate_reduce<1>(v, 0u, sh_f);
     const float var = v[0] / (float)(n - 1);  // n = 1: NaN, as torch.std
     tau = mean - __builtin_sqrtf(var);
   }
-  // per block (one wave per block, lanes over heads): any head retained,
-  // head-mean zeta, largest bound, beta = max_h qmax_h sqrt(E) / sqrt(d)
+  // per block (one 16-lane row per block, lanes over heads; a wave per block
+  // left half its lanes idle at 32 heads and cost 1 us per 16 blocks): any
+  // head retained, head-mean zeta, largest bound, beta = max_h qmax_h sqrt(E)
+  // / sqrt(d)
+  const int j = tid & 15, row = tid >> 4;
+  constexpr int kRows = 64;
+  auto row_max = [](float x) {
+    x = fmaxf(x, xpair<8>(x));
+    x = fmaxf(x, xpair<4>(x));
+    x = fmaxf(x, xpair<2>(x));
+    return fmaxf(x, xpair<1>(x));
+  };
   const float isd = 1.0f / __builtin_sqrtf((float)d);
   struct Blk {
     bool any;
@@ -382,22 +582,24 @@ __global__ __launch_bounds__(1024) void compact_gate_kernel(const float* mb, con
   auto block_stats = [&](int b) {
     bool any = false;
     float zsum = 0.f, bmx = -__builtin_inff(), beta = -__builtin_inff();
-    for (int h = lane; h < H; h += 64) {
-      const float m = mb[(int64_t)b * H + h], z = zeta[(int64_t)b * H + h];
+    for (int h = j; h < H; h += 16) {
+      const float m = mb_at((int64_t)b * H + h), z = zeta_at((int64_t)b * H + h);
       any = any || (m >= tau && z <= zeta_max);
       zsum += z;
       bmx = fmaxf(bmx, m);
-      beta = fmaxf(beta, qmax[h] * __builtin_sqrtf(fmaxf(energy[(int64_t)b * H + h], 0.f)) * isd);
+      beta = fmaxf(beta, qmax_at(h) * __builtin_sqrtf(fmaxf(energy_at((int64_t)b * H + h), 0.f)) * isd);
     }
-    return Blk{__ballot(any) != 0, wave_sum(zsum) / (float)H, wave_max(bmx), wave_max(beta)};
+    return Blk{((__ballot(any) >> (lane & 48)) & 0xFFFFu) != 0, row16_sum(zsum) / (float)H, row_max(bmx),
+               row_max(beta)};
   };
   // r1: zeta sum, retained (sums); -zeta min, zeta max, best retained bound (maxima)
   float r1[5] = {0.f, 0.f, -__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
-  for (int b = wave; b < nb; b += kGateWaves) {
+  for (int b = row; b < nb; b += kRows) {
     const Blk k = block_stats(b);
-    for (int t = lane; t < tiles_per_block; t += 64) tile_mask[(int64_t)b * tiles_per_block + t] = k.any ? 1 : 0;
-    if (lane == 0) {
-      unified[b] = k.any ? 1 : 0;
+    if (!cache_blk)
+      for (int t = j; t < tiles_per_block; t += 16) tile_mask[(int64_t)b * tiles_per_block + t] = k.any ? 1 : 0;
+    if (j == 0) {
+      if (!cache_blk) unified[b] = k.any ? 1 : 0;
       if (cache_blk) {
         sh_any[b] = k.any ? 1 : 0;
         sh_za[b] = k.za;
@@ -411,6 +613,10 @@ __global__ __launch_bounds__(1024) void compact_gate_kernel(const float* mb, con
     }
   }
   gate_reduce<5>(r1, 0x1Cu, sh_f);  // its barriers also publish sh_any / sh_za / sh_beta
+  if (cache_blk) {
+    for (int b = tid; b < nb; b += 1024) unified[b] = sh_any[b];
+    for (int64_t t = tid; t < (int64_t)nb * tiles_per_block; t += 1024) tile_mask[t] = sh_any[t / tiles_per_block];
+  }
   const float zmean = r1[0] / (float)nb;
   const float retained = r1[1];
   const float zmin = -r1[2], zmx = r1[3];
@@ -427,9 +633,9 @@ __global__ __launch_bounds__(1024) void compact_gate_kernel(const float* mb, con
   if (cache_blk) {
     for (int b = tid; b < nb; b += 1024) regime(sh_any[b] != 0, sh_za[b], sh_beta[b]);
   } else {
-    for (int b = wave; b < nb; b += kGateWaves) {
+    for (int b = row; b < nb; b += kRows) {
       const Blk k = block_stats(b);
-      if (lane == 0) regime(k.any, k.za, k.beta);
+      if (j == 0) regime(k.any, k.za, k.beta);
     }
   }
   gate_reduce<3>(r2, 0u, sh_f);
@@ -567,7 +773,7 @@ int launch_spectrum(const SpecArgs& a, hipStream_t s) {
   else if (a.d == 64)
     hipLaunchKernelGGL((block_spectrum_kernel<DT, 64>), dim3(a.H, a.nb), dim3(kSpThreads), 0, s, a);
   else
-    hipLaunchKernelGGL((block_spectrum_kernel<DT, 0>), dim3(a.H, a.nb), dim3(kSpThreads), 0, s, a);
+    hipLaunchKernelGGL(block_spectrum_any_kernel<DT>, dim3(a.H, a.nb), dim3(kSpThreads), 0, s, a);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? OC_OK : hip_fail(e, "block-spectrum launch");
 }
@@ -630,8 +836,9 @@ extern "C" int oc_compact_gate(const float* max_bound, const float* zeta, const 
   if (!max_bound || !zeta || !energy || !q_norm_max || !block_mask || !tile_mask || !stats)
     return fail(OC_ERR_INVALID, "NULL pointer");
   if (num_blocks < 1 || num_heads < 1 || head_dim < 1 || tiles_per_block < 1) return fail(OC_ERR_INVALID, "bad sizes");
-  hipLaunchKernelGGL(compact_gate_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, max_bound, zeta, energy,
-                     q_norm_max, num_blocks, num_heads, head_dim, (float)tau, tau_auto, (float)zeta_max,
+  const bool staged = (int64_t)num_blocks * num_heads <= kGateLds && num_heads <= kGateHeads;
+  hipLaunchKernelGGL(staged ? compact_gate_kernel<true> : compact_gate_kernel<false>, dim3(1), dim3(1024), 0,
+                     (hipStream_t)stream, max_bound, zeta, energy, q_norm_max, num_blocks, num_heads, head_dim, (float)tau, tau_auto, (float)zeta_max,
                      (float)underflow, tiles_per_block, block_mask, tile_mask, stats);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? OC_OK : hip_fail(e, "compact-gate launch");

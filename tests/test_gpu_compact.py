@@ -79,6 +79,32 @@ def test_block_spectra_vs_oracle(dtype, d):
     assert (z[[1, 3]] > 100).all() and (z[[0, 2, 4]] < 1).all()
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("Sq,q_dtype,shift", [(1, "bf16", 0), (33, "f32", 0), (70, "f16", 0), (17, "bf16", 1)])
+def test_block_spectra_query_groups(dtype, d, Sq, q_dtype, shift):
+    """Counts of queries around the groups of 16 and 32 a workgroup takes at
+    once, q of another dtype than K, and q rows that 16-byte loads cannot take
+    (shifted by one element); a constant block has E_low = 0 exactly."""
+    from orthocache_gpu import _launch as X
+    H, nb = 3, 3
+    k = _keys(nb, H, d, {1}, seed=d + Sq, dtype=dtype)
+    k[512:1024, 1] = torch.randn(d, generator=torch.Generator().manual_seed(2)).to(TD[dtype])
+    g = torch.Generator().manual_seed(Sq)
+    q = torch.randn((Sq * H * d + shift,), generator=g).to(TD[q_dtype]).to(DEV)[shift:].view(Sq, H, d)
+    print(f"spectra {dtype} d={d} Sq={Sq} q {q_dtype} shift={shift}", flush=True)
+    got = X.block_spectra(k.to(DEV), q, want_bounds=True, want_mean=True, want_qnorm=True)
+    ref = O.block_spectra(np64(k), np64(q))
+    for name in ("e_low", "e_mid", "e_high", "e_ac", "energy", "block_mean"):
+        np.testing.assert_allclose(np64(got[name]), ref[name], rtol=1e-5, atol=1e-6, err_msg=name)
+    assert (got["e_low"][1, 1] == 0).item() and (got["e_high"][1, 1] == 0).item()
+    # a bound is a sum of d products and ||q|| sqrt(E): relative to the larger of the two
+    scale = np.abs(ref["bounds"]).max()
+    np.testing.assert_allclose(np64(got["bounds"]), ref["bounds"], rtol=1e-5, atol=1e-5)
+    np.testing.assert_allclose(np64(got["max_bound"]), ref["bounds"].max(0), rtol=1e-5, atol=2e-6 * scale)
+    np.testing.assert_allclose(np64(got["q_norm_max"]), np.linalg.norm(np64(q), axis=-1).max(0), rtol=1e-6)
+
+
 def test_stream_compact_and_spectral_api():
     from orthocache_gpu import spectral_energy as SE
     from orthocache_gpu.adaptive_attention import stream_compact
@@ -148,6 +174,13 @@ def test_compact_gate_kernel_vs_oracle(nb, H):
             assert s[i] == pytest.approx(ref[key], rel=1e-5), key
         if nb > 1:
             assert s[2] == pytest.approx(ref["zeta_std"], rel=1e-4)
+
+
+@pytest.mark.parametrize("nb,H", [(67, 17), (130, 1), (64, 32), (2051, 2)])
+def test_compact_gate_rows_of_blocks(nb, H):
+    """Blocks around the 64 taken at once, heads around a row's 16, and more
+    blocks than the per-block results held in LDS (2048)."""
+    test_compact_gate_kernel_vs_oracle(nb, H)
 
 
 def _gap_tau(vals):
