@@ -182,6 +182,13 @@ class KVLayout:
         return d
 
 
+def distinct_rows(t: torch.Tensor, dim: int) -> torch.Tensor:
+    """t itself, or a copy when the tokens along dim share memory (an expanded
+    K or V): the kernels bound a tile's reads by its tokens times their stride,
+    and what lies beyond reads as zeros."""
+    return t.contiguous() if t.shape[dim] > 1 and t.stride(dim) < t.shape[-1] else t
+
+
 def rows_layout(keys: torch.Tensor, values: Optional[torch.Tensor], partial_tail: bool = False,
                 tile_size: int = TILE_SIZE) -> KVLayout:
     """(rows, S, d) K/V views (last dimension contiguous, any other strides).
@@ -192,9 +199,9 @@ def rows_layout(keys: torch.Tensor, values: Optional[torch.Tensor], partial_tail
     if values is not None and values.shape != keys.shape:
         raise ValueError(f"keys {tuple(keys.shape)} and values {tuple(values.shape)} must have the same shape")
     keys, values = harmonize_kv(keys, values)
-    keys = last_dim_ready(keys, d)
+    keys = distinct_rows(last_dim_ready(keys, d), 1)
     if values is not None:
-        values = last_dim_ready(values, d)
+        values = distinct_rows(last_dim_ready(values, d), 1)
     kv = KVLayout(
         k=keys, v=values, head_dim=d, num_rows=rows, num_tiles=s_len // tile_size,
         k_row_stride=keys.stride(0), k_token_stride=keys.stride(1),
@@ -814,7 +821,11 @@ def attend_takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
     query block stages it through LDS).  Eight is what the decode kernels take
     in one pass over a head's K and V."""
     few = 8 if q.dtype == torch.float32 else 1
-    return (q.shape[0] > few and q.dtype == k.dtype == v.dtype and q.shape[2] in (64, 128)
+    # what oc_attend refuses (rows 2^22 elements or more apart, over 2^17 query
+    # blocks) stays on the decode kernels
+    fits = (k.stride(0) < 1 << 22 and v.stride(0) < 1 << 22
+            and q.shape[1] * ((q.shape[0] + 127) // 128) <= 1 << 17)
+    return (q.shape[0] > few and fits and q.dtype == k.dtype == v.dtype and q.shape[2] in (64, 128)
             and q.dtype in (torch.float32, torch.float16, torch.bfloat16) and 0 < k.shape[0] <= 1 << 20
             and q.shape[1:] == k.shape[1:] and k.shape == v.shape)
 
@@ -826,7 +837,7 @@ def attend(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out_dtype: torch.d
     up,), shared by the heads, 1 = attend."""
     device = require_gpu(q, k, v)
     Sq, H, d = q.shape
-    q, k, v = (ready16(t) for t in (q, k, v))
+    q, k, v = (ready16(t) for t in (q, distinct_rows(k, 0), distinct_rows(v, 0)))
     out = torch.empty((Sq, H, d), dtype=out_dtype, device=device)
     p = N.OcAttendParams()
     p.q, (p.q_stride_s, p.q_stride_h) = q.data_ptr(), q.stride()[:2]

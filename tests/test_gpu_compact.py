@@ -359,6 +359,25 @@ def test_attend_query_blocks(dtype, d, H, Sq, S, splits):
         assert_out(out, ref, dtype, f"attend {dtype} d={d} Sq={Sq} S={S} masked={m is not None}")
 
 
+@pytest.mark.parametrize("expanded", ["k", "v", "q"])
+@pytest.mark.parametrize("Sq", [1, 20])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_dense_forward_of_expanded_tensors(dtype, Sq, expanded):
+    """Tokens (or queries) that share one row of memory, on the decode kernels
+    (one query) and the query blocks: an expanded V was read as zeros."""
+    from orthocache_gpu.pipeline import orthocache_forward
+    H, S, d = 4, 256, 64
+    g = torch.Generator().manual_seed(9)
+    t = {n: torch.randn((s, H, d), generator=g).to(TD[dtype]).to(DEV) for n, s in (("q", Sq), ("k", S), ("v", S))}
+    t[expanded] = t[expanded][:1].expand(t[expanded].shape[0], H, d)
+    out, _ = orthocache_forward(t["q"], t["k"], t["v"], mode="dense")
+    q, k, v = (np64(t[n].contiguous()) for n in "qkv")
+    logits = np.einsum("qhd,khd->hqk", q, k) / np.sqrt(d)
+    p = np.exp(logits - logits.max(axis=2, keepdims=True))
+    ref = np.einsum("hqk,khd->qhd", p / p.sum(axis=2, keepdims=True), v)
+    assert_out(out, ref, dtype, f"dense forward {dtype} Sq={Sq} expanded {expanded}")
+
+
 @pytest.mark.parametrize("P", [1, 8, 9, 16, 17, 32, 33])
 @pytest.mark.parametrize("d", [4, 64, 96, 256])
 def test_merge_of_few_partials(P, d):
