@@ -46,6 +46,9 @@
  *   oc_row_norms + oc_kth_smallest <- torch.norm(q_group, dim=-1) and its
  *                      .median(dim=1) (perplexity_eval.py:454-456);
  *                      _compute_q_high_norm (perplexity_eval.py:547-573)
+ *   oc_prefill_gate <- the prefill branch's gate as a whole: q norms, median,
+ *                      K tile norms, compares, statistics and cache fill
+ *                      (perplexity_eval.py:447-497)
  *   oc_group_gate   <- the per-(kv head, tile) Cauchy-Schwarz compares of the
  *                      prefill and decode branches (perplexity_eval.py:476-491,
  *                      :639-657)
@@ -57,6 +60,8 @@
  *   oc_compact_gate  <- compute_multiband_mask, _compute_auto_tau, the zeta
  *                      statistics and classify_eviction as orthocache_forward
  *                      runs them (pipeline.py:458-527)
+ *   oc_attend        <- the attention over the retained (or all) blocks for a
+ *                      block of queries (pipeline.py:528-583)
  *   oc_block_regimes <- compute_block_beta + classify_eviction
  *                      (perfect_eviction.py:75-186)
  *   oc_device_props  <- torch.cuda.get_device_properties as _detect_gpu_profile
