@@ -523,7 +523,8 @@ def hook_decode(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, k_n
         return out.to(dt), stats
     rows = []
     for t in (key, value):
-        if t.stride(3) != 1 or (B > 1 and t.stride(0) != Hkv * t.stride(1)):
+        sb, sh, ss, sd = t.stride()  # ss < d: tokens that share memory (distinct_rows)
+        if sd != 1 or ss < d or (B > 1 and sb != Hkv * sh):
             t = t.contiguous()
         rows.append(t)
     key, value = rows

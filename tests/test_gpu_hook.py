@@ -544,3 +544,26 @@ def test_prefill_paired_windows_vs_oracle(dtype, d, S, masked):
                                            None if evict is None else evict.numpy())
     assert_out(out, ref, dtype, f"prefill paired {dtype} d={d} S={S} masked={masked}")
     np.testing.assert_allclose(np64(ent), ref_ent, atol=1e-4, rtol=1e-5)
+
+
+@pytest.mark.parametrize("expanded", ["k", "v", "overlapping"])
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+def test_hook_decode_of_tokens_that_share_memory(dtype, expanded):
+    """An expanded K or V (token stride 0), and tokens half a row apart: a
+    tile's reads are bounded by its tokens times their stride, so the decode
+    took what lies beyond as zeros."""
+    from orthocache_gpu import _launch as X
+    B, Hq, Hkv, d, S = 2, 4, 2, 64, 200
+    q, k, v = _qkv(B, Hq, Hkv, 1, S, d, dtype, seed=71)
+    if expanded == "k":
+        k = k[:, :, :1].expand(B, Hkv, S, d)
+    elif expanded == "v":
+        v = v[:, :, :1].expand(B, Hkv, S, d)
+    else:
+        k = torch.randn((B, Hkv, (S + 1) * d // 2), generator=torch.Generator().manual_seed(72)).to(TD[dtype]).to(DEV)
+        k = k.as_strided((B, Hkv, S, d), (k.stride(0), k.stride(1), d // 2, 1))
+    norms = torch.ones((Hkv, S // 64), device=DEV)
+    print(f"hook decode {dtype} expanded {expanded}", flush=True)
+    out, _ = X.hook_decode(q, k, v, norms, Hq // Hkv, 0.0, 8)
+    ref = O.hook_decode(np64(q), np64(k), np64(v), np64(norms), Hq // Hkv, 0.0)
+    assert_out(out, ref["out"], dtype, f"hook decode {dtype} expanded {expanded}")
