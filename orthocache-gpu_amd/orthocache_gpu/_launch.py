@@ -525,11 +525,12 @@ def hook_decode(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, k_n
     for t in (key, value):
         sb, sh, ss, sd = t.stride()  # ss < d: tokens that share memory (distinct_rows)
         if sd != 1 or ss < d or (B > 1 and sb != Hkv * sh):
-            t = t.contiguous()
+            # (contiguous() keeps the head stride of a single head as it is)
+            t = t.clone(memory_format=torch.contiguous_format)
         rows.append(t)
     key, value = rows
     if query.stride(3) != 1 or (B > 1 and query.stride(0) != Hq * query.stride(1)):
-        query = query.contiguous()
+        query = query.clone(memory_format=torch.contiguous_format)
     device = query.device
     if not (device.type == "cuda" and key.device == device and value.device == device and k_norms.device == device):
         require_gpu(query, key, value, k_norms)  # raises with the reason

@@ -567,3 +567,20 @@ def test_hook_decode_of_tokens_that_share_memory(dtype, expanded):
     out, _ = X.hook_decode(q, k, v, norms, Hq // Hkv, 0.0, 8)
     ref = O.hook_decode(np64(q), np64(k), np64(v), np64(norms), Hq // Hkv, 0.0)
     assert_out(out, ref["out"], dtype, f"hook decode {dtype} expanded {expanded}")
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_hook_decode_of_one_transposed_kv_head(dtype):
+    """K and V of a single head as a decoder layer's (B, S, 1, d) -> (B, 1, S,
+    d) views: torch calls them contiguous, with a head stride of d, and the
+    decode took the second batch element's rows one token after the first's."""
+    from orthocache_gpu import _launch as X
+    B, Hq, d, S = 3, 4, 64, 130
+    q, k, v = _qkv(B, Hq, 1, 1, S, d, dtype, seed=73)
+    k, v = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in (k, v))
+    assert k.stride(1) == d and k.is_contiguous()
+    norms = torch.ones((1, S // 64), device=DEV)
+    print(f"hook decode {dtype} one transposed kv head", flush=True)
+    out, _ = X.hook_decode(q, k, v, norms, Hq, 0.0, 8)
+    ref = O.hook_decode(np64(q), np64(k), np64(v), np64(norms), Hq, 0.0)
+    assert_out(out, ref["out"], dtype, f"hook decode {dtype} one transposed kv head")
