@@ -186,7 +186,7 @@ def distinct_rows(t: torch.Tensor, dim: int) -> torch.Tensor:
     """t itself, or a copy when the tokens along dim share memory (an expanded
     K or V): the kernels bound a tile's reads by its tokens times their stride,
     and what lies beyond reads as zeros."""
-    return t.contiguous() if t.shape[dim] > 1 and t.stride(dim) < t.shape[-1] else t
+    return t.clone(memory_format=torch.contiguous_format) if t.stride(dim) < t.shape[-1] else t
 
 
 def rows_layout(keys: torch.Tensor, values: Optional[torch.Tensor], partial_tail: bool = False,
@@ -230,8 +230,8 @@ def paged_layout(k_cache: torch.Tensor, v_cache: torch.Tensor, block_tables: tor
         raise ValueError("block_tables must be 2-D (num_seqs, max_blocks)")
     if not (keep_mixed and mixed_fp8k_bf16v(k_cache, v_cache)):
         k_cache, v_cache = harmonize_kv(k_cache, v_cache)
-    k_cache = last_dim_ready(k_cache, d)
-    v_cache = last_dim_ready(v_cache, d)
+    k_cache = distinct_rows(last_dim_ready(k_cache, d), 2)
+    v_cache = distinct_rows(last_dim_ready(v_cache, d), 2)
     if block_tables.dtype != torch.int32:
         block_tables = block_tables.to(torch.int32)
     if block_tables.stride(-1) != 1:

@@ -829,3 +829,30 @@ def test_headline_size_properties(gate):
     ref = torch.einsum("hgs,hsd->hgd", torch.softmax(logits, dim=-1), v64).reshape(Hkv * G, d)
     assert_out(o1, ref.cpu().numpy(), "bf16", f"headline B=1 {gate} single pass")
     assert_out(o2, ref.cpu().numpy(), "bf16", f"headline B=1 {gate} cached")
+
+
+@pytest.mark.parametrize("expanded", ["k", "v"])
+@pytest.mark.parametrize("mode", ["single_pass", "cached"])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_paged_pool_whose_tokens_share_memory(dtype, mode, expanded):
+    """A pool with one stored token a page (token stride 0) gives what the
+    same pool laid out gives: a 16-token block's reads are bounded by its
+    tokens times their stride, so an expanded V was read as zeros."""
+    from orthocache_gpu import fused_orthocache_attention_paged
+    from orthocache_gpu.triton_kernels.paged_eviction import score_paged_tiles
+    from orthocache_gpu.workloads import make_q
+    B, hkv, bs, d, pages = 2, 2, 16, 128, 20
+    g = torch.Generator().manual_seed(3)
+    pool = {n: torch.randn((B * pages, hkv, bs, d), generator=g).to(TORCH_DT[dtype]).to(DEV) for n in "kv"}
+    bt = torch.randperm(B * pages, generator=g).view(B, pages).to(torch.int32).to(DEV)
+    q = make_q(B * hkv, 4, d, seed=4).to(TORCH_DT[dtype]).to(DEV).view(B, hkv * 4, d)
+    one = pool[expanded][:, :, :1].expand(-1, -1, bs, -1)
+    res = []
+    for t in (one, one.contiguous()):
+        k, v = (t if n == expanded else pool[n] for n in "kv")
+        sc = score_paged_tiles(k, bt) if mode == "cached" else None
+        print(f"paged expanded {expanded} {mode} {dtype}", flush=True)
+        out, m = fused_orthocache_attention_paged(q, k, v, bt, 5.0, num_query_groups=4, mode=mode, score_cache=sc)
+        res.append((out, m["tiles_retained"], None if sc is None else sc.e_low))
+    assert torch.equal(res[0][0], res[1][0]) and res[0][1] == res[1][1] > 0
+    assert res[0][0].abs().amax() > 0 and (mode != "cached" or torch.equal(res[0][2], res[1][2]))
