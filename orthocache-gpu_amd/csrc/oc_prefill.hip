@@ -1777,6 +1777,7 @@ extern "C" int oc_prefill_gate(const oc_prefill_gate_params* p, void* stream) {
     if ((st * es) % 16) return fail(OC_ERR_INVALID, "q/k strides must be multiples of 16 bytes");
   if (((uintptr_t)p->q | (uintptr_t)p->k) % 16) return fail(OC_ERR_INVALID, "q/k not 16-byte aligned");
   if (p->k_stride_s * es * 64 > 0x7FFFFFFF) return fail(OC_ERR_UNSUPPORTED, "token stride too large");
+  if (p->k_stride_s < p->head_dim) return fail(OC_ERR_INVALID, "token stride smaller than head_dim");
   if (p->cache && p->cache_stride < T) return fail(OC_ERR_INVALID, "norm cache rows of %lld, %d tiles",
                                                    (long long)p->cache_stride, T);
   // one workgroup per 4 tiles, and per 64 query rows at the least

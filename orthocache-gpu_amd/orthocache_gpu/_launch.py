@@ -889,7 +889,7 @@ def prefill_gate(q: torch.Tensor, k: torch.Tensor, tau_norm: float, norm_scale: 
                  stats_out: Optional[torch.Tensor] = None, cache: Optional[torch.Tensor] = None,
                  valid_tiles: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
     """oc_prefill_gate over q (B, Hq, Sq, d) and k (B, Hkv, Skv, d), both as
-    `ready16` gives them: (evict mask uint8 (B, Hkv, T), norm_scale times
+    `ready16` (k also `distinct_rows`) gives them: (evict mask uint8 (B, Hkv, T), norm_scale times
     the band norms float32 (B, Hkv, T)) of the T = Skv // 64 complete
     tiles.  stats_out: contiguous float32 (B, Hkv, 3) for group_gate's
     statistics; cache (>= Hkv, >= T) float32 with contiguous rows and
@@ -926,7 +926,7 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, tile
     the stream's workspace)."""
     device = check_prefill(q, k, v)
     B, Hq, Sq, d = q.shape
-    q, k, v = (ready16(t) for t in (q, k, v))
+    q, k, v = ready16(q), distinct_rows(ready16(k), 2), distinct_rows(ready16(v), 2)
     Hkv, Skv = k.shape[1], k.shape[2]
     out = torch.empty((B, Hq, Sq, d), dtype=q.dtype, device=device)
     ent = torch.empty((B, Hq, Sq), dtype=torch.float32, device=device) if want_entropy else None

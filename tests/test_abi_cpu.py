@@ -120,6 +120,37 @@ def test_hook_entry_point_argument_checks():
                            None) == N.OC_ERR_INVALID
 
 
+def test_prefill_gate_argument_checks():
+    """oc_prefill_gate validates on the host; none of these calls launches."""
+    import ctypes
+    from orthocache_gpu import _native as N
+    L = N.lib()
+    assert L.oc_prefill_gate_params_bytes() == ctypes.sizeof(N.OcPrefillGateParams)
+
+    def refused(code, text, **change):
+        p = N.OcPrefillGateParams()
+        p.q = p.k = p.q_norms = p.k_norms = p.mask = 256
+        p.dtype, p.batch, p.num_q_heads, p.num_kv_heads, p.q_len, p.kv_len, p.head_dim = N.OC_BF16, 1, 4, 2, 8, 128, 64
+        for x in ("q_stride_b", "q_stride_h", "q_stride_s", "k_stride_b", "k_stride_h", "k_stride_s"):
+            setattr(p, x, 64)
+        for x, y in change.items():
+            setattr(p, x, y)
+        assert L.oc_prefill_gate(ctypes.byref(p), None) == code and text in L.oc_last_error(), change
+
+    assert L.oc_prefill_gate(None, None) == N.OC_ERR_INVALID
+    refused(N.OC_ERR_UNSUPPORTED, b"dtype", dtype=N.OC_FP8_E4M3FN)
+    refused(N.OC_ERR_UNSUPPORTED, b"head_dim", head_dim=32)
+    refused(N.OC_ERR_INVALID, b"sizes", q_len=0)
+    refused(N.OC_ERR_INVALID, b"multiple", num_q_heads=5)
+    refused(N.OC_ERR_INVALID, b"NULL", mask=None)
+    refused(N.OC_ERR_INVALID, b"16 bytes", q_stride_s=65)
+    refused(N.OC_ERR_INVALID, b"aligned", k=264)
+    refused(N.OC_ERR_UNSUPPORTED, b"stride too large", k_stride_s=1 << 24)
+    refused(N.OC_ERR_INVALID, b"smaller than head_dim", k_stride_s=0)
+    refused(N.OC_ERR_INVALID, b"smaller than head_dim", k_stride_s=56)
+    refused(N.OC_ERR_INVALID, b"norm cache", cache=256, cache_stride=1)
+
+
 def test_spectra_argument_checks():
     import ctypes
     from orthocache_gpu import _native as N

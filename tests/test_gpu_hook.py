@@ -584,3 +584,28 @@ def test_hook_decode_of_one_transposed_kv_head(dtype):
     out, _ = X.hook_decode(q, k, v, norms, Hq, 0.0, 8)
     ref = O.hook_decode(np64(q), np64(k), np64(v), np64(norms), Hq, 0.0)
     assert_out(out, ref["out"], dtype, f"hook decode {dtype} one transposed kv head")
+
+
+@pytest.mark.parametrize("expanded", ["k", "v"])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("S", [40, 200])  # dense below one tile
+def test_hook_prefill_of_tokens_that_share_memory(dtype, expanded, S):
+    """An expanded K or V: its tile norms (and the norm cache) were those of
+    zeros, and the attention refused the call after that."""
+    from orthocache_gpu.model_hook import OrthoCache_GQA_Attention
+    from orthocache_gpu.norm_cache import SpectralNormCache
+    B, Hq, Hkv, d = 2, 4, 2, 64
+    q, k, v = _qkv(B, Hq, Hkv, S, S, d, dtype, seed=74)
+    if expanded == "k":
+        k = k[:, :, :1].expand(B, Hkv, S, d)
+    else:
+        v = v[:, :, :1].expand(B, Hkv, S, d)
+    hook = OrthoCache_GQA_Attention(tau=-1.0)
+    hook.norm_cache = SpectralNormCache(Hkv, 8, torch.device(DEV))
+    print(f"hook prefill {dtype} expanded {expanded} S={S}", flush=True)
+    out = hook.orthocache_attention(q, k, v, Hq // Hkv)
+    ref, _ = O.hook_causal_attention(np64(q), np64(k), np64(v), Hq // Hkv)
+    assert_out(out, ref, dtype, f"hook prefill {dtype} expanded {expanded} S={S}")
+    T = S // 64
+    want = O.hook_tile_norms(np64(k))[B - 1]  # equal tokens: no high-band energy, but for the rounding of the sums
+    np.testing.assert_allclose(np64(hook.norm_cache.cache[:, :T]), want, rtol=4 * 2.0 ** -23, atol=1e-4)
