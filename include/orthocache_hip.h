@@ -132,6 +132,9 @@ extern "C" {
  *                     + (t % block_size) * k_token_stride + c) elements.
  *             Block ids outside [0, num_blocks) make the call fail with
  *             OC_ERR_INVALID reported through `error_flag`.
+ *             Token strides are at least head_dim; a smaller one (tokens that
+ *             share memory) is OC_ERR_INVALID, but in the portable kernels
+ *             and, on pages, wherever the matrix cores are not used.
  * lengths:    NULL, or int32 token counts indexed by r / rows_per_length;
  *             a row has ceil(len/64) tiles (at most num_tiles).  Full tiles
  *             are scored; a partial tail tile is always retained and its

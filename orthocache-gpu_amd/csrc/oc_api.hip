@@ -151,6 +151,18 @@ static int fill_kv(const oc_kv_desc* kv, DecodeArgs& a, bool allow_dq = false) {
   return OC_OK;
 }
 
+// The tuned kernels on contiguous rows, and the matrix-core decode on pages,
+// bound a tile's (a 16-token block's) reads by its tokens times their stride,
+// so tokens that share memory would be read as zeros there.  (The portable
+// kernels, and the tuned ones elsewhere on pages, address each token and take
+// any stride.)
+static int check_token_strides(const oc_kv_desc* kv, bool with_v) {
+  if (kv->num_rows == 0 || kv->num_tiles == 0) return OC_OK;
+  if (kv->k_token_stride < kv->head_dim || (with_v && kv->v_token_stride < kv->head_dim))
+    return fail(OC_ERR_INVALID, "token stride smaller than head_dim");
+  return OC_OK;
+}
+
 template <int DT>
 hipError_t launch_decode(const DecodeArgs& a, int head_dim, int gt, int gchunks, hipStream_t st);
 template <int DT>
@@ -812,6 +824,7 @@ static int decode_impl(const oc_decode_params* p, void* ws, size_t ws_bytes, voi
     const int dt = p->kv.dtype;
     const bool mq = (dt == OC_BF16 && p->q_dtype == OC_BF16) || (dt == OC_F16 && p->q_dtype == OC_F16) ||
                     (dt == OC_FP8_E4M3FN && p->q_dtype == OC_BF16);
+    if ((!a.paged || (mq && a.bs_log2 >= 4)) && (rc = check_token_strides(&p->kv, true))) return rc;
     const bool cached_gate = p->mode == OC_MODE_CACHED && p->gate != OC_GATE_NONE;
     const bool q16 = aligned(p->q, 16) && (a.q_row_stride % 16) == 0;
     a.fast = (mq && (!a.paged || a.bs_log2 >= 4) && gchunks == 1 && q16 &&
@@ -1026,6 +1039,7 @@ extern "C" int oc_score_tiles(const oc_kv_desc* kv, double zeta_max, float* e_lo
   a.q_dtype = OC_F32;
   a.t0 = 0;
   a.tcnt = kv->num_tiles;
+  if (!a.paged && !generic_shape(kv->head_dim, a.ts) && (rc = check_token_strides(kv, false))) return rc;
   if ((int64_t)kv->num_rows * kv->num_tiles == 0) return OC_OK;
   const hipError_t e = generic_shape(kv->head_dim, a.ts) ? gen_launch_score(kv->dtype, a, kv->head_dim, (hipStream_t)stream)
                                                          : dispatch_score(kv->dtype, a, kv->head_dim, (hipStream_t)stream);
@@ -1049,6 +1063,7 @@ extern "C" int oc_score_tile_range(const oc_kv_desc* kv, int32_t first_tile, int
   a.q_dtype = OC_F32;
   a.t0 = first_tile;
   a.tcnt = count;
+  if (!a.paged && !generic_shape(kv->head_dim, a.ts) && (rc = check_token_strides(kv, false))) return rc;
   if ((int64_t)kv->num_rows * count == 0) return OC_OK;
   const hipError_t e = generic_shape(kv->head_dim, a.ts) ? gen_launch_score(kv->dtype, a, kv->head_dim, (hipStream_t)stream)
                                                          : dispatch_score(kv->dtype, a, kv->head_dim, (hipStream_t)stream);
@@ -1075,6 +1090,7 @@ extern "C" int oc_band_norms(const oc_kv_desc* kv, int32_t first_tile, int32_t c
   a.o_norm = out;
   a.o_stride = out_row_stride;
   a.o_valid = valid_tiles;
+  if (!a.paged && (rc = check_token_strides(kv, false))) return rc;
   if ((int64_t)kv->num_rows * count == 0) return OC_OK;
   const hipError_t e = dispatch_band(kv->dtype, a, kv->head_dim, (hipStream_t)stream);
   return e == hipSuccess ? OC_OK : hip_fail(e, "band-norm launch");
@@ -1094,6 +1110,7 @@ extern "C" int oc_fwht_tiles(const oc_kv_desc* kv, float* out, void* stream) {
     const hipError_t e = gen_launch_score(kv->dtype, a, kv->head_dim, (hipStream_t)stream);
     return e == hipSuccess ? OC_OK : hip_fail(e, "fwht launch");
   }
+  if (!a.paged && (rc = check_token_strides(kv, false))) return rc;
   const hipError_t e = dispatch_fwht(kv->dtype, a, kv->head_dim, (hipStream_t)stream);
   return e == hipSuccess ? OC_OK : hip_fail(e, "fwht launch");
 }

@@ -120,6 +120,53 @@ def test_hook_entry_point_argument_checks():
                            None) == N.OC_ERR_INVALID
 
 
+def test_token_strides_below_head_dim_are_refused():
+    """Every entry point whose kernel bounds its reads by tokens x stride
+    refuses tokens that share memory (they would be read as zeros); none of
+    these calls launches."""
+    import ctypes
+    from orthocache_gpu import _native as N
+    L = N.lib()
+    for dtype in (N.OC_BF16, N.OC_F32):
+        for d, portable in ((128, 0), (64, 0), (256, 1), (32, 1)):
+            for ks, vs in ((0, d), (d // 2, d), (d, 0), (-d, d)):
+                p = N.OcDecodeParams()
+                kv = p.kv
+                kv.k = kv.v = 256
+                kv.dtype, kv.head_dim, kv.num_rows, kv.num_tiles = dtype, d, 2, 4
+                kv.k_row_stride = kv.v_row_stride = 256 * d
+                kv.k_token_stride, kv.v_token_stride = ks, vs
+                p.q, p.q_dtype, p.G, p.q_row_stride, p.num_splits = 256, dtype, 1, d, 2
+                p.out, p.out_dtype, p.out_row_stride = 256, dtype, d
+                p.mode, p.gate = N.OC_MODE_CACHED, N.OC_GATE_NONE
+                p.workspace, p.workspace_bytes = 256, 1 << 30
+                if dtype == N.OC_BF16 or not portable:  # float32 at 32 and 256 runs the portable kernels
+                    assert L.oc_decode(ctypes.byref(p), None) == N.OC_ERR_INVALID
+                    assert b"smaller than head_dim" in L.oc_last_error(), (dtype, d, ks, vs)
+                if portable or ks == d:
+                    continue
+                for rc in (L.oc_score_tiles(ctypes.byref(kv), 5.0, 256, 256, None, None, 4, None),
+                           L.oc_score_tile_range(ctypes.byref(kv), 0, 1, 5.0, 256, 256, None, None, 4, None),
+                           L.oc_band_norms(ctypes.byref(kv), 0, 1, 48, 64, 256, 4, None, None),
+                           L.oc_fwht_tiles(ctypes.byref(kv), 256, None)):
+                    assert rc == N.OC_ERR_INVALID
+                    assert b"smaller than head_dim" in L.oc_last_error()
+    # on pages: the matrix-core decode (16-token pages, q of K's 16-bit type)
+    p = N.OcDecodeParams()
+    kv = p.kv
+    kv.k = kv.v = kv.block_tables = 256
+    kv.dtype, kv.head_dim, kv.num_rows, kv.num_tiles = N.OC_F16, 128, 2, 4
+    kv.paged, kv.block_size, kv.num_kv_heads, kv.num_blocks, kv.bt_stride = 1, 16, 2, 32, 16
+    kv.k_block_stride = kv.v_block_stride = 4096
+    kv.k_head_stride = kv.v_head_stride = 2048
+    kv.k_token_stride, kv.v_token_stride = 128, 0
+    p.q, p.q_dtype, p.G, p.q_row_stride, p.num_splits = 256, N.OC_F16, 1, 128, 2
+    p.out, p.out_dtype, p.out_row_stride = 256, N.OC_F16, 128
+    p.workspace, p.workspace_bytes = 256, 1 << 30
+    assert L.oc_decode(ctypes.byref(p), None) == N.OC_ERR_INVALID
+    assert b"smaller than head_dim" in L.oc_last_error()
+
+
 def test_prefill_gate_argument_checks():
     """oc_prefill_gate validates on the host; none of these calls launches."""
     import ctypes
