@@ -373,6 +373,11 @@ typedef struct oc_prefill_params {
 
 int oc_prefill_attention(const oc_prefill_params* p, void* stream);
 
+/* what oc_prefill_attention would return for p before its launch: a caller
+ * that launches other work first (the hook's gate, which fills the norm
+ * cache) learns of a refusal before it.  No reference counterpart. */
+int oc_prefill_check(const oc_prefill_params* p);
+
 /* bytes of workspace that lets oc_prefill_attention split the longest causal
  * windows (0: this call would not split).  No reference counterpart. */
 size_t oc_prefill_workspace_size(const oc_prefill_params* p);

@@ -1555,7 +1555,9 @@ bool pf_plan(const oc_prefill_params* p, PfPlan* pl) {
 
 using namespace oc;
 
-extern "C" int oc_prefill_attention(const oc_prefill_params* p, void* stream) {
+// Everything that oc_prefill_attention refuses; *split: the call has a
+// workspace and splits its longest windows by *pl.
+static int prefill_check(const oc_prefill_params* p, PfPlan* pl, bool* split) {
   if (!p) return fail(OC_ERR_INVALID, "NULL params");
   if (!p->q || !p->k || !p->v || !p->out) return fail(OC_ERR_INVALID, "NULL tensor pointer");
   if (!pf_float_dtype(p->dtype)) return fail(OC_ERR_UNSUPPORTED, "prefill dtype %d (float32, float16, bfloat16)",
@@ -1582,6 +1584,30 @@ extern "C" int oc_prefill_attention(const oc_prefill_params* p, void* stream) {
   if (p->tile_mask && p->tile_mask_cols < p->kv_len / 64)
     return fail(OC_ERR_INVALID, "tile_mask has %d columns, kv_len needs %d", p->tile_mask_cols, p->kv_len / 64);
   if (p->batch == 0 || p->num_q_heads == 0 || p->q_len == 0) return OC_OK;
+  *split = p->workspace && pf_plan(p, pl);
+  if (*split) {
+    const size_t need = kPfCounterBytes + pl->part_bytes + 256;
+    if (p->workspace_bytes < need)
+      return fail(OC_ERR_WORKSPACE, "prefill workspace of %zu bytes needed, %zu given", need, p->workspace_bytes);
+  }
+  const int64_t items = *split ? pl->nitems : (p->q_len + kPfRows - 1) / kPfRows;
+  if (items * p->batch * p->num_q_heads > 0x7FFFFFFF) return fail(OC_ERR_UNSUPPORTED, "too many query blocks");
+  return OC_OK;
+}
+
+extern "C" int oc_prefill_check(const oc_prefill_params* p) {
+  PfPlan pl;
+  bool split = false;
+  return prefill_check(p, &pl, &split);
+}
+
+extern "C" int oc_prefill_attention(const oc_prefill_params* p, void* stream) {
+  PfPlan pl;
+  bool split = false;
+  const int rc = prefill_check(p, &pl, &split);
+  if (rc) return rc;
+  if (p->batch == 0 || p->num_q_heads == 0 || p->q_len == 0) return OC_OK;
+  const int es = p->dtype == OC_F32 ? 4 : 2;
   PrefillArgs a{};
   a.q = (const char*)p->q;
   a.k = (const char*)p->k;
@@ -1598,26 +1624,17 @@ extern "C" int oc_prefill_attention(const oc_prefill_params* p, void* stream) {
   a.entropy = p->entropy;
   a.qblocks = (p->q_len + kPfRows - 1) / kPfRows;
   a.o_vec = ((uintptr_t)p->out | (uintptr_t)a.o_sb | (uintptr_t)a.o_sh | (uintptr_t)a.o_ss) % 8 == 0;
-  int64_t items = a.qblocks;
   a.rev = pf_first_fill(p, a.qblocks);
-  if (p->workspace) {
-    PfPlan pl;
-    if (pf_plan(p, &pl)) {
-      const size_t need = kPfCounterBytes + pl.part_bytes + 256;
-      if (p->workspace_bytes < need)
-        return fail(OC_ERR_WORKSPACE, "prefill workspace of %zu bytes needed, %zu given", need, p->workspace_bytes);
-      char* w = (char*)(((uintptr_t)p->workspace + 255) & ~(uintptr_t)255);
-      a.ctr = (int32_t*)w;
-      a.part = (float*)(w + kPfCounterBytes);
-      a.nitems = pl.nitems;
-      a.q0 = pl.q0;
-      a.ctr_stride = pl.ctr_stride;
-      std::copy(pl.items, pl.items + pl.nitems, a.items);
-      items = pl.nitems;
-    }
+  if (split) {
+    char* w = (char*)(((uintptr_t)p->workspace + 255) & ~(uintptr_t)255);
+    a.ctr = (int32_t*)w;
+    a.part = (float*)(w + kPfCounterBytes);
+    a.nitems = pl.nitems;
+    a.q0 = pl.q0;
+    a.ctr_stride = pl.ctr_stride;
+    std::copy(pl.items, pl.items + pl.nitems, a.items);
   }
-  const int64_t blocks = items * a.B * a.Hq;
-  if (blocks > 0x7FFFFFFF) return fail(OC_ERR_UNSUPPORTED, "too many query blocks");
+  const int64_t blocks = (int64_t)(split ? pl.nitems : a.qblocks) * a.B * a.Hq;
   const hipStream_t s = (hipStream_t)stream;
   switch (p->dtype) {
     case OC_F32: return launch_prefill_d<OC_F32>(a, p->head_dim, s, (unsigned)blocks);

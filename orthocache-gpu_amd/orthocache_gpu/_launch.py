@@ -10,7 +10,7 @@ from __future__ import annotations
 import ctypes
 import threading
 from dataclasses import dataclass
-from typing import Dict, Optional, Tuple
+from typing import Callable, Dict, Optional, Tuple
 
 import numpy as np
 import torch
@@ -887,13 +887,15 @@ def norm_cache_ready(cache: torch.Tensor, valid_tiles: torch.Tensor, device: tor
 
 def prefill_gate(q: torch.Tensor, k: torch.Tensor, tau_norm: float, norm_scale: float, *,
                  stats_out: Optional[torch.Tensor] = None, cache: Optional[torch.Tensor] = None,
-                 valid_tiles: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+                 valid_tiles: Optional[torch.Tensor] = None, mask: Optional[torch.Tensor] = None
+                 ) -> Tuple[torch.Tensor, torch.Tensor]:
     """oc_prefill_gate over q (B, Hq, Sq, d) and k (B, Hkv, Skv, d), both as
     `ready16` (k also `distinct_rows`) gives them: (evict mask uint8 (B, Hkv, T), norm_scale times
     the band norms float32 (B, Hkv, T)) of the T = Skv // 64 complete
     tiles.  stats_out: contiguous float32 (B, Hkv, 3) for group_gate's
     statistics; cache (>= Hkv, >= T) float32 with contiguous rows and
-    valid_tiles int32 take the last batch element's norms."""
+    valid_tiles int32 take the last batch element's norms.  mask: where the
+    flags go, a new tensor by default."""
     device = require_gpu(q, k)
     B, Hq, Sq, d = q.shape
     Hkv, T = k.shape[1], k.shape[2] // TILE_SIZE
@@ -905,7 +907,8 @@ def prefill_gate(q: torch.Tensor, k: torch.Tensor, tau_norm: float, norm_scale: 
     p.norm_scale, p.tau_norm = norm_scale, tau_norm
     qn = torch.empty((B, Hq, Sq), dtype=torch.float32, device=device)
     kn = torch.empty((B, Hkv, T), dtype=torch.float32, device=device)
-    mask = torch.empty((B, Hkv, T), dtype=torch.uint8, device=device)
+    if mask is None:
+        mask = torch.empty((B, Hkv, T), dtype=torch.uint8, device=device)
     p.q_norms, p.k_norms, p.mask, p.gate_stats = qn.data_ptr(), kn.data_ptr(), mask.data_ptr(), _ptr(stats_out)
     if cache is not None:
         p.cache, p.cache_stride, p.valid_tiles = cache.data_ptr(), cache.stride(0), _ptr(valid_tiles)
@@ -915,7 +918,8 @@ def prefill_gate(q: torch.Tensor, k: torch.Tensor, tau_norm: float, norm_scale: 
 
 
 def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, tile_mask: Optional[torch.Tensor] = None,
-                      scale: Optional[float] = None, want_entropy: bool = False, split: bool = True
+                      scale: Optional[float] = None, want_entropy: bool = False, split: bool = True,
+                      before_launch: Optional[Callable[[], None]] = None
                       ) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
     """oc_prefill_attention: causal GQA attention of q (B, Hq, Sq, d) over k, v
     (B, Hkv, Skv, d) (last dimensions contiguous, other strides free),
@@ -923,7 +927,9 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, tile
     Returns (out (B, Hq, Sq, d) in q's dtype, entropy float32 (B, Hq, Sq) or
     None).  split: let the library run the longest causal windows as two
     workgroups each when the call fits the device in one round (it then uses
-    the stream's workspace)."""
+    the stream's workspace).  before_launch() is called once nothing but the
+    launch can fail any more: what it launches comes before the attention on
+    the stream, and may write tile_mask."""
     device = check_prefill(q, k, v)
     B, Hq, Sq, d = q.shape
     q, k, v = ready16(q), distinct_rows(ready16(k), 2), distinct_rows(ready16(v), 2)
@@ -954,6 +960,9 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, tile
         if nws:
             ws = workspace(device, stream, nws)
             p.workspace, p.workspace_bytes = ws.data_ptr(), ws.numel()
+        if before_launch is not None:
+            N.check("oc_prefill_check", lib.oc_prefill_check(ctypes.byref(p)))
+            before_launch()
         N.check("oc_prefill_attention", lib.oc_prefill_attention(ctypes.byref(p), ctypes.c_void_p(stream)))
     return out, ent
 

@@ -160,6 +160,7 @@ SIGNATURES = {
     "oc_group_gate": (_i32, [_p, _i32, _i32, _i32, _i32, _p, _i64, _i64, _i32, _i32, ctypes.c_double, _i32, _p,
                              _i64, _i64, _p, _p, _p]),
     "oc_prefill_attention": (_i32, [ctypes.POINTER(OcPrefillParams), _p]),
+    "oc_prefill_check": (_i32, [ctypes.POINTER(OcPrefillParams)]),
     "oc_prefill_workspace_size": (ctypes.c_size_t, [ctypes.POINTER(OcPrefillParams)]),
     "oc_prefill_params_bytes": (ctypes.c_size_t, []),
     "oc_attend": (_i32, [ctypes.POINTER(OcAttendParams), _p]),

@@ -263,13 +263,21 @@ class OrthoCache_GQA_Attention:
         # the norms ||(H64 K_t)[48:64]||_F of every complete tile, per q head
         # the lower median over positions of ||q||_2, the group's max, the
         # gate and its statistics, and the norm cache
+        # (which is written only once the attention has nothing left to refuse)
         in_kernel = nc is not None and X.norm_cache_ready(nc.cache, nc.valid_tiles, key.device)
         dev = self.stats.ring_rows(query.device, (B, Hkv, 3))
-        evict, kn = X.prefill_gate(query, key, tau * TILE * d, _HOOK_NORM_SCALE, stats_out=dev,
+        evict = torch.empty((B, Hkv, T), dtype=torch.uint8, device=query.device)
+        kn = None
+
+        def gate():
+            nonlocal kn
+            _, kn = X.prefill_gate(query, key, tau * TILE * d, _HOOK_NORM_SCALE, stats_out=dev, mask=evict,
                                    cache=nc.cache if in_kernel else None,
                                    valid_tiles=nc.valid_tiles if in_kernel else None)
+
         want_entropy = self.governor is not None and hasattr(self.governor, 'set_entropy')
-        out, ent = X.prefill_attention(query, key, value, tile_mask=evict, want_entropy=want_entropy)
+        out, ent = X.prefill_attention(query, key, value, tile_mask=evict, want_entropy=want_entropy,
+                                       before_launch=gate)
         if nc is not None:
             if not in_kernel:
                 # the reference's per-batch loop writes cache[kv_h, t] for every batch

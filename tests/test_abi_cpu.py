@@ -120,6 +120,32 @@ def test_hook_entry_point_argument_checks():
                            None) == N.OC_ERR_INVALID
 
 
+def test_prefill_check_refuses_what_the_attention_refuses():
+    """oc_prefill_check gives oc_prefill_attention's answer (and message)
+    without its launch; a call it accepts is only checked here."""
+    import ctypes
+    from orthocache_gpu import _native as N
+    L = N.lib()
+    good = dict(q=256, k=256, v=256, out=256, dtype=N.OC_F32, head_dim=64, batch=1, num_q_heads=4, num_kv_heads=2,
+                q_len=8, kv_len=200, q_stride_s=64, k_stride_s=64, v_stride_s=64, tile_mask=256, tile_mask_cols=3)
+
+    def params(**change):
+        p = N.OcPrefillParams()
+        for x, y in {**good, **change}.items():
+            setattr(p, x, y)
+        return ctypes.byref(p)
+
+    assert L.oc_prefill_check(params()) == N.OC_OK
+    assert L.oc_prefill_check(None) == N.OC_ERR_INVALID
+    for change in (dict(v=None), dict(head_dim=32), dict(dtype=N.OC_FP8_E4M3FN), dict(num_kv_heads=3),
+                   dict(k_stride_s=65), dict(k=264), dict(out=264), dict(v_stride_s=1 << 23), dict(v_stride_s=0),
+                   dict(tile_mask_cols=2), dict(num_q_heads=1 << 30, num_kv_heads=1, q_len=1 << 20)):
+        rc = L.oc_prefill_check(params(**change))
+        msg = L.oc_last_error()
+        assert rc != N.OC_OK and msg, change
+        assert L.oc_prefill_attention(params(**change), None) == rc and L.oc_last_error() == msg, change
+
+
 def test_token_strides_below_head_dim_are_refused():
     """Every entry point whose kernel bounds its reads by tokens x stride
     refuses tokens that share memory (they would be read as zeros); none of

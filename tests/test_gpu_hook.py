@@ -609,3 +609,29 @@ def test_hook_prefill_of_tokens_that_share_memory(dtype, expanded, S):
     T = S // 64
     want = O.hook_tile_norms(np64(k))[B - 1]  # equal tokens: no high-band energy, but for the rounding of the sums
     np.testing.assert_allclose(np64(hook.norm_cache.cache[:, :T]), want, rtol=4 * 2.0 ** -23, atol=1e-4)
+
+
+@pytest.mark.parametrize("own_rows", [True, False], ids=["in kernel", "copied"])
+def test_refused_prefill_leaves_the_norm_cache(own_rows):
+    """A prefill that the attention refuses (a V whose tile spans 2 GiB) has
+    written nothing to the norm cache; the same call with a V that it takes
+    fills it."""
+    from orthocache_gpu import _native as N
+    from orthocache_gpu.model_hook import OrthoCache_GQA_Attention
+    from orthocache_gpu.norm_cache import SpectralNormCache
+    S, d = 64, 64
+    q, k, v = _qkv(1, 2, 1, S, S, d, "f32", seed=75)
+    far = 1 << 23
+    v_far = torch.empty((S * far,), device=DEV).as_strided((1, 1, S, d), (S * far, S * far, far, 1))
+    hook = OrthoCache_GQA_Attention(tau=-1.0)
+    nc = hook.norm_cache = SpectralNormCache(1, 4, torch.device(DEV))
+    nc.cache.fill_(-7.0)
+    if not own_rows:  # another type than the gate writes itself
+        nc.valid_tiles = nc.valid_tiles.long()
+    with pytest.raises(N.OrthoCacheHIPError, match="token stride too large"):
+        hook.orthocache_attention(q, k, v_far, 2)
+    assert (nc.cache == -7).all() and not nc.valid_tiles.any() and not nc.is_populated
+    assert hook.stats['layers_processed'] == 0
+    hook.orthocache_attention(q, k, v, 2)
+    np.testing.assert_allclose(np64(nc.cache[:, 0]), O.hook_tile_norms(np64(k))[0, :, 0], rtol=4 * 2.0 ** -23)
+    assert nc.valid_tiles.tolist() == [1] and nc.is_populated
