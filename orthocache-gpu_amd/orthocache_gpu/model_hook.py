@@ -265,7 +265,9 @@ class OrthoCache_GQA_Attention:
         # gate and its statistics, and the norm cache
         # (which is written only once the attention has nothing left to refuse)
         in_kernel = nc is not None and X.norm_cache_ready(nc.cache, nc.valid_tiles, key.device)
-        dev = self.stats.ring_rows(query.device, (B, Hkv, 3))
+        # the call's own statistics: a slot of the shared ring is free again at
+        # the next fold, which does not wait for other streams or a graph's replays
+        dev = torch.empty((B, Hkv, 3), dtype=torch.float32, device=query.device)
         evict = torch.empty((B, Hkv, T), dtype=torch.uint8, device=query.device)
         kn = None
 

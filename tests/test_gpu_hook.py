@@ -635,3 +635,25 @@ def test_refused_prefill_leaves_the_norm_cache(own_rows):
     hook.orthocache_attention(q, k, v, 2)
     np.testing.assert_allclose(np64(nc.cache[:, 0]), O.hook_tile_norms(np64(k))[0, :, 0], rtol=4 * 2.0 ** -23)
     assert nc.valid_tiles.tolist() == [1] and nc.is_populated
+
+
+def test_prefill_statistics_are_not_shared_between_streams():
+    """A prefill's statistics are its own until they are folded: another
+    stream's fold in between, and the calls after it, leave them alone (a
+    ring slot was given to the next call while the first could still write)."""
+    from orthocache_gpu.model_hook import OrthoCache_GQA_Attention
+    hook = OrthoCache_GQA_Attention(tau=-1.0)
+    q, k, v = _qkv(1, 4, 2, 128, 128, 64, "f32", seed=76)
+    rows = []
+    defer = hook.stats.defer
+    hook.stats.defer = lambda fold, dev, run=None: (rows.append(dev), defer(fold, dev, run))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        hook.orthocache_attention(q, k, v, 2)
+    assert hook.stats['layers_processed'] == 1  # folds on this stream
+    hook.orthocache_attention(q, k, v, 2)
+    hook.orthocache_attention(q, k, v, 2)
+    assert len({r.data_ptr() for r in rows}) == 3
+    torch.cuda.synchronize()
+    assert all(torch.equal(r, rows[0]) for r in rows)
