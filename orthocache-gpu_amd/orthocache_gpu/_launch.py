@@ -822,12 +822,13 @@ def attend_takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
     and 123 / 102 for nine (the decode holds a float32 tile in registers, the
     query block stages it through LDS).  Eight is what the decode kernels take
     in one pass over a head's K and V."""
-    few = 8 if q.dtype == torch.float32 else 1
+    if q.shape[0] <= (8 if q.dtype == torch.float32 else 1):
+        return False
     # what oc_attend refuses (rows 2^22 elements or more apart, over 2^17 query
     # blocks) stays on the decode kernels
     fits = (k.stride(0) < 1 << 22 and v.stride(0) < 1 << 22
             and q.shape[1] * ((q.shape[0] + 127) // 128) <= 1 << 17)
-    return (q.shape[0] > few and fits and q.dtype == k.dtype == v.dtype and q.shape[2] in (64, 128)
+    return (fits and q.dtype == k.dtype == v.dtype and q.shape[2] in (64, 128)
             and q.dtype in (torch.float32, torch.float16, torch.bfloat16) and 0 < k.shape[0] <= 1 << 20
             and q.shape[1:] == k.shape[1:] and k.shape == v.shape)
 

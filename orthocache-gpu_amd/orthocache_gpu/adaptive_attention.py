@@ -61,9 +61,10 @@ def attend_tiles(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, 
     seq_q, nh, hd = q.shape
     if tokens > k_cache.shape[0] or tokens % X.TILE_SIZE:
         raise ValueError(f"{tokens} tokens: more than the cache holds or not whole tiles")
-    if X.attend_takes(q, k_cache[:tokens], v_cache[:tokens]):
-        return X.attend(q, k_cache[:tokens], v_cache[:tokens], torch.bfloat16, tile_mask=tile_mask.reshape(-1))
-    kv = X.rows_layout(k_cache[:tokens].permute(1, 0, 2), v_cache[:tokens].permute(1, 0, 2))
+    k, v = k_cache[:tokens], v_cache[:tokens]
+    if X.attend_takes(q, k, v):
+        return X.attend(q, k, v, torch.bfloat16, tile_mask=tile_mask.reshape(-1))
+    kv = X.rows_layout(k.permute(1, 0, 2), v.permute(1, 0, 2))
     tm = tile_mask.reshape(1, -1).expand(nh, -1)
     out = torch.empty((seq_q, nh, hd), dtype=torch.bfloat16, device=q.device)
     if seq_q == 1:  # the decode's output rows are this call's
