@@ -103,9 +103,10 @@ def last_dim_ready(t: torch.Tensor, head_dim: int) -> torch.Tensor:
     contiguous copy (the reference wrappers always copy, fused_eviction.py:636-638)."""
     es = t.element_size()
     al = _kv_align(head_dim, es)
-    ok = t.stride(-1) == 1 and _aligned(t, al)
+    *outer, last = t.stride()
+    ok = last == 1 and _aligned(t, al)
     if ok:
-        for s in t.stride()[:-1]:
+        for s in outer:
             if (s * es) % al:
                 ok = False
     return t if ok else t.contiguous()
@@ -189,6 +190,17 @@ def distinct_rows(t: torch.Tensor, dim: int) -> torch.Tensor:
     return t.clone(memory_format=torch.contiguous_format) if t.stride(dim) < t.shape[-1] else t
 
 
+def _row_strides(t: torch.Tensor, d: int) -> tuple:
+    """K or V (..., tokens, d) as last_dim_ready and distinct_rows give it, and
+    its strides but the last (taken once: every decode call comes here)."""
+    t = last_dim_ready(t, d)
+    *outer, tok, _ = t.stride()
+    if tok < d:
+        t = distinct_rows(t, t.dim() - 2)
+        *outer, tok, _ = t.stride()
+    return t, *outer, tok
+
+
 def rows_layout(keys: torch.Tensor, values: Optional[torch.Tensor], partial_tail: bool = False,
                 tile_size: int = TILE_SIZE) -> KVLayout:
     """(rows, S, d) K/V views (last dimension contiguous, any other strides).
@@ -199,14 +211,13 @@ def rows_layout(keys: torch.Tensor, values: Optional[torch.Tensor], partial_tail
     if values is not None and values.shape != keys.shape:
         raise ValueError(f"keys {tuple(keys.shape)} and values {tuple(values.shape)} must have the same shape")
     keys, values = harmonize_kv(keys, values)
-    keys = distinct_rows(last_dim_ready(keys, d), 1)
+    keys, k_row, k_tok = _row_strides(keys, d)
+    v_row = v_tok = 0
     if values is not None:
-        values = distinct_rows(last_dim_ready(values, d), 1)
+        values, v_row, v_tok = _row_strides(values, d)
     kv = KVLayout(
         k=keys, v=values, head_dim=d, num_rows=rows, num_tiles=s_len // tile_size,
-        k_row_stride=keys.stride(0), k_token_stride=keys.stride(1),
-        v_row_stride=0 if values is None else values.stride(0),
-        v_token_stride=0 if values is None else values.stride(1), tile_size=tile_size)
+        k_row_stride=k_row, k_token_stride=k_tok, v_row_stride=v_row, v_token_stride=v_tok, tile_size=tile_size)
     if partial_tail and s_len % tile_size:
         kv.num_tiles += 1
         kv.num_tokens = s_len
@@ -230,18 +241,17 @@ def paged_layout(k_cache: torch.Tensor, v_cache: torch.Tensor, block_tables: tor
         raise ValueError("block_tables must be 2-D (num_seqs, max_blocks)")
     if not (keep_mixed and mixed_fp8k_bf16v(k_cache, v_cache)):
         k_cache, v_cache = harmonize_kv(k_cache, v_cache)
-    k_cache = distinct_rows(last_dim_ready(k_cache, d), 2)
-    v_cache = distinct_rows(last_dim_ready(v_cache, d), 2)
+    k_cache, k_block, k_head, k_tok = _row_strides(k_cache, d)
+    v_cache, v_block, v_head, v_tok = _row_strides(v_cache, d)
     if block_tables.dtype != torch.int32:
         block_tables = block_tables.to(torch.int32)
     if block_tables.stride(-1) != 1:
         block_tables = block_tables.contiguous()
     return KVLayout(
         k=k_cache, v=v_cache, head_dim=d, num_rows=block_tables.shape[0] * hkv, num_tiles=num_tiles,
-        k_token_stride=k_cache.stride(2), v_token_stride=v_cache.stride(2),
+        k_token_stride=k_tok, v_token_stride=v_tok,
         paged=True, block_size=bs, num_kv_heads=hkv, block_tables=block_tables, num_blocks=nb,
-        k_block_stride=k_cache.stride(0), k_head_stride=k_cache.stride(1),
-        v_block_stride=v_cache.stride(0), v_head_stride=v_cache.stride(1),
+        k_block_stride=k_block, k_head_stride=k_head, v_block_stride=v_block, v_head_stride=v_head,
         rows_per_length=hkv, tile_size=tile_size)
 
 
