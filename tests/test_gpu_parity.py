@@ -852,7 +852,9 @@ def test_paged_pool_whose_tokens_share_memory(dtype, mode, expanded):
         k, v = (t if n == expanded else pool[n] for n in "kv")
         sc = score_paged_tiles(k, bt) if mode == "cached" else None
         print(f"paged expanded {expanded} {mode} {dtype}", flush=True)
-        out, m = fused_orthocache_attention_paged(q, k, v, bt, 5.0, num_query_groups=4, mode=mode, score_cache=sc)
+        # tokens equal within 16 have no energy in Walsh rows 1..7: zeta is
+        # e_high / 1e-6, at most 64 d max(k)^2 / 1e-6 < 1e12, and every tile stays
+        out, m = fused_orthocache_attention_paged(q, k, v, bt, 1e12, num_query_groups=4, mode=mode, score_cache=sc)
         res.append((out, m["tiles_retained"], None if sc is None else sc.e_low))
     assert torch.equal(res[0][0], res[1][0]) and res[0][1] == res[1][1] > 0
     assert res[0][0].abs().amax() > 0 and (mode != "cached" or torch.equal(res[0][2], res[1][2]))
