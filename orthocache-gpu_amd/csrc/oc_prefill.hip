@@ -1785,16 +1785,16 @@ extern "C" int oc_prefill_gate(const oc_prefill_gate_params* p, void* stream) {
     return fail(OC_ERR_INVALID, "bad sizes");
   if (p->num_q_heads % p->num_kv_heads) return fail(OC_ERR_INVALID, "num_q_heads %d not a multiple of num_kv_heads %d",
                                                     p->num_q_heads, p->num_kv_heads);
-  const int T = p->kv_len / 64;
-  if (p->batch == 0 || p->num_q_heads == 0 || T == 0) return OC_OK;
-  if (!p->q || !p->k || !p->q_norms || !p->k_norms || !p->mask) return fail(OC_ERR_INVALID, "NULL pointer");
+  const int T = p->kv_len / 64;  // with no complete tile the query norms and the statistics are still written
+  if (p->batch == 0 || p->num_q_heads == 0) return OC_OK;
+  if (!p->q || !p->q_norms || (T && (!p->k || !p->k_norms || !p->mask))) return fail(OC_ERR_INVALID, "NULL pointer");
   const int es = p->dtype == OC_F32 ? 4 : 2;
   const int64_t strides[] = {p->q_stride_b, p->q_stride_h, p->q_stride_s, p->k_stride_b, p->k_stride_h, p->k_stride_s};
   for (int64_t st : strides)
     if ((st * es) % 16) return fail(OC_ERR_INVALID, "q/k strides must be multiples of 16 bytes");
   if (((uintptr_t)p->q | (uintptr_t)p->k) % 16) return fail(OC_ERR_INVALID, "q/k not 16-byte aligned");
   if (p->k_stride_s * es * 64 > 0x7FFFFFFF) return fail(OC_ERR_UNSUPPORTED, "token stride too large");
-  if (p->k_stride_s < p->head_dim) return fail(OC_ERR_INVALID, "token stride smaller than head_dim");
+  if (T && p->k_stride_s < p->head_dim) return fail(OC_ERR_INVALID, "token stride smaller than head_dim");
   if (p->cache && p->cache_stride < T) return fail(OC_ERR_INVALID, "norm cache rows of %lld, %d tiles",
                                                    (long long)p->cache_stride, T);
   // one workgroup per 4 tiles, and per 64 query rows at the least

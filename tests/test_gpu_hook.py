@@ -657,3 +657,22 @@ def test_prefill_statistics_are_not_shared_between_streams():
     assert len({r.data_ptr() for r in rows}) == 3
     torch.cuda.synchronize()
     assert all(torch.equal(r, rows[0]) for r in rows)
+
+
+def test_prefill_gate_with_no_complete_tile():
+    """Fewer keys than a tile: the query norms, the group norm and the
+    statistics are those of the entry points it stands for (no evicted tile,
+    a K maximum of -inf); the norm cache is left alone."""
+    from orthocache_gpu import _launch as X
+    B, Hq, Hkv, d, S = 2, 6, 2, 64, 63
+    q, k, _ = _qkv(B, Hq, Hkv, S, S, d, "bf16", seed=77)
+    st = torch.full((B, Hkv, 3), 5.0, device=DEV)
+    cache = torch.full((Hkv, 4), -5.0, device=DEV)
+    valid = torch.tensor([0, 3], dtype=torch.int32, device=DEV)
+    mask, kn = X.prefill_gate(q, k, 1.0, 8.0, stats_out=st, cache=cache, valid_tiles=valid)
+    assert mask.shape == kn.shape == (B, Hkv, 0)
+    qn = O.torch_lower_median(np.linalg.norm(np64(q), axis=-1)).reshape(B, Hkv, Hq // Hkv).max(axis=2)
+    st = st.cpu().numpy()
+    np.testing.assert_allclose(st[:, :, 1], qn, rtol=8 * 2.0 ** -23)
+    assert (st[:, :, 0] == 0).all() and np.isneginf(st[:, :, 2]).all()
+    assert (cache == -5).all() and valid.tolist() == [0, 3]
