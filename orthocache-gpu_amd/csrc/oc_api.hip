@@ -464,19 +464,6 @@ extern "C" int oc_dequant_fp8(const void* src, int64_t n, float scale, int32_t o
   return e == hipSuccess ? OC_OK : hip_fail(e, "dequant launch");
 }
 
-// CU count of the current device, cached per device index.
-static int device_cus() {
-  static int cache[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!cache[dev]) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cache[dev] = n;
-  }
-  return cache[dev];
-}
-
 // query heads per decode workgroup for G heads per kv row (chunks of up to 8)
 static int heads_per_group(const oc_decode_params* p) {
   const int G = p->G;

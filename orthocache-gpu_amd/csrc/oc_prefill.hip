@@ -901,10 +901,7 @@ void launch_attend(const AttendArgs& a, int d, unsigned blocks, hipStream_t s) {
 constexpr int kAtPerCu = 2, kAtMinTiles = 4;
 
 int attend_shares(const oc_attend_params* p) {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    cus = 256;
+  const int64_t cus = device_cus();
   const int64_t blocks = (int64_t)p->num_heads * ((p->q_len + kPfRows - 1) / kPfRows);
   const int64_t tiles = (p->kv_len + 63) / 64;
   if (p->num_splits > 0) return (int)std::max<int64_t>(1, std::min<int64_t>({p->num_splits, tiles, 8192}));
@@ -1446,13 +1443,6 @@ int pf_slots_t() {
   return per_cu[dev] > 0 ? per_cu[dev] * cus[dev] : 0;
 }
 
-int pf_cus() {
-  int dev = 0, c = 0;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return 0;
-  return c;
-}
-
 int pf_slots(int dtype, int d) {
   switch (dtype) {
     case OC_F32: return d == 64 ? pf_slots_t<OC_F32, 64>() : pf_slots_t<OC_F32, 128>();
@@ -1470,8 +1460,8 @@ int pf_slots(int dtype, int d) {
 // 64 in bfloat16 50.5 / 43.5 / 31.7 against 49.3 / 38.3 / 31.2.)
 int pf_first_fill(const oc_prefill_params* p, int items) {
   const int64_t nbh = (int64_t)p->batch * p->num_q_heads;
-  const int slots = pf_slots(p->dtype, p->head_dim), cus = pf_cus();
-  if (cus <= 0 || slots < 2 * cus || nbh * items > 2 * (int64_t)cus || nbh > cus) return items;
+  const int slots = pf_slots(p->dtype, p->head_dim), cus = device_cus();
+  if (slots < 2 * cus || nbh * items > 2 * (int64_t)cus || nbh > cus) return items;
   return (int)std::min<int64_t>(items, cus / nbh);
 }
 
@@ -1506,7 +1496,7 @@ bool pf_plan(const oc_prefill_params* p, PfPlan* pl) {
   // x 1531 35.2 / 37.3 and 42.0 / 45.3; 16 heads x 3579 in bfloat16 97 / 101).
   // head_dim 64 keeps the split (32 x 2043: float32 156 / 155, bfloat16 47.1 /
   // 47.7; 8 heads x 8187: 576 / 589 and 150 / 177).
-  const int64_t cus = pf_cus();
+  const int64_t cus = device_cus();
   if (p->head_dim == 128 && nbh * 8 >= cus && nbh * qblocks * 8 >= 14 * cus && pf_first_fill(p, qblocks) < qblocks)
     return false;
   const int off = p->kv_len - p->q_len;
