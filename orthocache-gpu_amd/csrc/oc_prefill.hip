@@ -1149,13 +1149,18 @@ __device__ __forceinline__ void select_rows(const float* x, int64_t stride, int 
   }
 }
 
-// One workgroup per row (select_rows).
-__global__ __launch_bounds__(kSelThreads) void kth_smallest_kernel(const float* x, int64_t n, int64_t row_stride,
-                                                                   int64_t k, float* out) {
+// `per` rows per workgroup (select_rows; sel_rows chooses); ONE: one, which the
+// compiler then knows (8 rows of a million values: 720 us against 751).
+template <bool ONE>
+__global__ __launch_bounds__(kSelThreads) void kth_smallest_kernel(const float* x, int64_t rows, int64_t n,
+                                                                   int64_t row_stride, int64_t k, int per,
+                                                                   float* out) {
   __shared__ SelLds s;
-  __shared__ float sel;
-  select_rows(x + (int64_t)blockIdx.x * row_stride, 0, 1, n, (uint64_t)k, s, &sel);
-  if (threadIdx.x == 0) out[blockIdx.x] = sel;
+  __shared__ float sel[kSelRows];
+  const int64_t r0 = ONE ? blockIdx.x : (int64_t)blockIdx.x * per;
+  const int nr = ONE ? 1 : (int)min((int64_t)per, rows - r0);
+  select_rows(x + r0 * row_stride, ONE ? 0 : row_stride, nr, n, (uint64_t)k, s, sel);
+  if ((int)threadIdx.x < nr) out[r0 + threadIdx.x] = sel[threadIdx.x];
 }
 
 // The group norm of G per-head norms: their max (NaN-propagating) or the
@@ -1451,6 +1456,20 @@ int pf_slots(int dtype, int d) {
   }
 }
 
+// Rows per workgroup of kth_smallest_kernel: more than one as long as about
+// two workgroups a CU remain and a row's values still fit its waves'
+// registers.  A workgroup's fixed cost (a histogram of 1024 bins per row, the
+// barriers) is then shared.  us for one row a workgroup / this rule: 1024 rows
+// of 16 values 20 / 12, 4096 of 64 73 / 14, of 2048 84 / 21, 65536 of 16 1120 /
+// 190, of 1024 1211 / 227 (256 threads a row with one radix over all 32 bits:
+// 39, 65, 78, 724, 781).
+int sel_rows(int64_t rows, int64_t n) {
+  const int64_t cus = device_cus();
+  int per = 1;
+  while (per < kSelRows && rows >= 4 * cus * per && n * (2 * per) <= (int64_t)kSelHeld * kSelThreads) per *= 2;
+  return per;
+}
+
 // When a call's workgroups all fit the device at once, at most two to a CU,
 // the first n of a head's `items` work items (longest first) go one to each CU
 // and the rest join them: shortest first, so that every CU gets about the same
@@ -1741,8 +1760,9 @@ extern "C" int oc_kth_smallest(const float* x, int64_t rows, int64_t n, int64_t 
   if (rows < 0 || n < 1 || k < 0 || k >= n || row_stride < n) return fail(OC_ERR_INVALID, "bad sizes (k must be < n)");
   if (rows > 0x7FFFFFFF) return fail(OC_ERR_UNSUPPORTED, "too many rows");
   if (rows == 0) return OC_OK;
-  hipLaunchKernelGGL(kth_smallest_kernel, dim3((unsigned)rows), dim3(kSelThreads), 0, (hipStream_t)stream, x, n, row_stride,
-                     k, out);
+  const int per = sel_rows(rows, n);
+  hipLaunchKernelGGL(per == 1 ? kth_smallest_kernel<true> : kth_smallest_kernel<false>, dim3((unsigned)((rows + per - 1) / per)), dim3(kSelThreads), 0,
+                     (hipStream_t)stream, x, rows, n, row_stride, k, per, out);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? OC_OK : hip_fail(e, "select launch");
 }

@@ -676,3 +676,18 @@ def test_prefill_gate_with_no_complete_tile():
     np.testing.assert_allclose(st[:, :, 1], qn, rtol=8 * 2.0 ** -23)
     assert (st[:, :, 0] == 0).all() and np.isneginf(st[:, :, 2]).all()
     assert (cache == -5).all() and valid.tolist() == [0, 3]
+
+
+@pytest.mark.parametrize("rows,n", [(1024, 1), (1025, 65), (2051, 8192), (4099, 64), (4096, 2049)])
+def test_selection_of_many_short_rows(rows, n):
+    """Several rows per workgroup (2, 4 and 8, the last workgroup part full)
+    and the lengths at which a row no longer fits its waves' registers."""
+    from orthocache_gpu import _launch as X
+    g = torch.Generator().manual_seed(rows + n)
+    x = torch.randn((rows, n), generator=g).abs()
+    x[::3] = x[::3].mul(4).round()  # ties
+    x[1::5] = 2.5
+    srt = np.sort(x.numpy(), axis=1)
+    print(f"selection {rows} rows of {n}", flush=True)
+    for k in sorted({0, (n - 1) // 2, n - 1}):
+        assert np.array_equal(X.kth_smallest(x.to(DEV), k).cpu().numpy(), srt[:, k]), k
