@@ -282,6 +282,23 @@ __global__ __launch_bounds__(kSpThreads, 4) void block_spectrum_kernel(const Spe
     r4[j] = sh_sum[0][j];
     for (int w = 1; w < WAVES; ++w) r4[j] += sh_sum[w][j];
   }
+  if (__builtin_isnan(r4[2])) {
+    // K that is not finite (uniform over the workgroup): the transform's rows
+    // 1..63 of a column with one infinity are all infinite, of one with more,
+    // or with a NaN, some are NaN; without its mean both are NaN
+    int* cnt = reinterpret_cast<int*>(&sh_col[0][0]);
+    if (tid < D) cnt[tid] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < COLS; ++c)
+#pragma unroll
+      for (int i = 0; i < TPT; ++i)
+        if (!__builtin_isfinite(z0[i][c])) atomicAdd(&cnt[cg * COLS + c], __builtin_isnan(z0[i][c]) ? 2 : 1);
+    __syncthreads();
+    bool nan = false;
+    for (int c = 0; c < D; ++c) nan = nan || cnt[c] > 1;
+    r4[2] = nan ? __builtin_nanf("") : __builtin_inff();
+  }
   const int64_t o = (int64_t)blk * a.H + h;
   const float s_ac = sp_write(a, o, r4[0], r4[1], r4[2] * 0.125f, r4[3], tid == 0);  // 64 / 512
   if (!a.q) return;

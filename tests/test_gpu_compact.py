@@ -394,3 +394,31 @@ def test_merge_of_few_partials(P, d):
     got = X.lse_merge(m.to(DEV), l.to(DEV), acc.to(DEV))
     # P float32 products per value, weights exp() of differences up to about 40
     np.testing.assert_allclose(np64(got), ref, atol=1e-5, rtol=1e-5)
+
+
+@pytest.mark.parametrize("dtype,d", _SPEC_GRID)
+def test_block_spectra_of_keys_that_are_not_finite(dtype, d):
+    """One infinity in a column makes every band infinite and the block's bounds
+    with it; two in a column, or a NaN, make the transform's sums NaN.  (E_low from the
+    columns less their means made NaN of a single infinity.)"""
+    from orthocache_gpu import _launch as X
+    k = _keys(4, 2, d, {1}, seed=d + 1, dtype=dtype)
+    k[5, 0, 3] = math.inf                            # block 0, head 0: one
+    k[9, 1, 0] = -math.inf                           # head 1: one in each of two columns
+    k[200, 1, d - 1] = math.inf
+    k[512 + 7, 0, 1], k[512 + 100, 0, 1] = math.inf, math.inf  # block 1: two in one column
+    k[512 + 7, 1, 1], k[512 + 71, 1, 1] = math.inf, math.inf   # of one position of two chunks
+    k[1024 + 40, 0, 2] = math.nan                    # block 2: a NaN, and a finite head beside it
+    q = torch.randn((3, 2, d), generator=torch.Generator().manual_seed(1)).to(TD[dtype])
+    print(f"spectra not finite {dtype} d={d}", flush=True)
+    got = X.block_spectra(k.to(DEV), q.to(DEV), want_bounds=True, want_mean=True)
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = O.block_spectra(np64(k), np64(q))
+    assert np.isposinf(ref["e_low"][0]).all() and np.isnan(ref["e_low"][1, 0]) and np.isposinf(ref["e_low"][1, 1])
+    for name in ("e_mid", "e_high"):  # by Parseval over the positions: infinite where the transform's rows are NaN
+        assert np.isnan(ref[name][1, 0]) and not np.isfinite(np64(got[name])[1, 0])
+        ref[name][1, 0] = np64(got[name])[1, 0]
+    for name in ("e_low", "e_mid", "e_high", "e_ac", "energy", "block_mean"):
+        np.testing.assert_allclose(np64(got[name]), ref[name], rtol=1e-5, atol=1e-6, err_msg=name)
+    for b in (0, 2, 3):  # (block 1's energy is NaN, which its bounds take as none)
+        np.testing.assert_allclose(np64(got["bounds"])[:, b], ref["bounds"][:, b], rtol=1e-5, atol=1e-5)
