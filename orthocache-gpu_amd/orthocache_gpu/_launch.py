@@ -850,7 +850,7 @@ def attend(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out_dtype: torch.d
     up,), shared by the heads, 1 = attend."""
     device = require_gpu(q, k, v)
     Sq, H, d = q.shape
-    q, k, v = (ready16(t) for t in (q, distinct_rows(k, 0), distinct_rows(v, 0)))
+    q, k, v = ready16(q), ready16(k, 0), ready16(v, 0)
     out = torch.empty((Sq, H, d), dtype=out_dtype, device=device)
     p = N.OcAttendParams()
     p.q, (p.q_stride_s, p.q_stride_h) = q.data_ptr(), q.stride()[:2]
@@ -901,8 +901,8 @@ def prefill_gate(q: torch.Tensor, k: torch.Tensor, tau_norm: float, norm_scale: 
                  valid_tiles: Optional[torch.Tensor] = None, mask: Optional[torch.Tensor] = None
                  ) -> Tuple[torch.Tensor, torch.Tensor]:
     """oc_prefill_gate over q (B, Hq, Sq, d) and k (B, Hkv, Skv, d), both as
-    `ready16` (k also `distinct_rows`) gives them: (evict mask uint8 (B, Hkv, T), norm_scale times
-    the band norms float32 (B, Hkv, T)) of the T = Skv // 64 complete
+    `ready16` gives them (k with its token dimension): (evict mask uint8 (B,
+    Hkv, T), norm_scale times the band norms float32 (B, Hkv, T)) of the T = Skv // 64 complete
     tiles.  stats_out: contiguous float32 (B, Hkv, 3) for group_gate's
     statistics; cache (>= Hkv, >= T) float32 with contiguous rows and
     valid_tiles int32 take the last batch element's norms.  mask: where the
@@ -943,7 +943,7 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, tile
     the stream, and may write tile_mask."""
     device = check_prefill(q, k, v)
     B, Hq, Sq, d = q.shape
-    q, k, v = ready16(q), distinct_rows(ready16(k), 2), distinct_rows(ready16(v), 2)
+    q, k, v = ready16(q), ready16(k, 2), ready16(v, 2)
     Hkv, Skv = k.shape[1], k.shape[2]
     out = torch.empty((B, Hq, Sq, d), dtype=q.dtype, device=device)
     ent = torch.empty((B, Hq, Sq), dtype=torch.float32, device=device) if want_entropy else None
@@ -978,13 +978,21 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, tile
     return out, ent
 
 
-def ready16(t: torch.Tensor) -> torch.Tensor:
-    """t itself when its last dimension is contiguous and its base and every
-    other stride are 16-byte aligned (the kernels' vector loads), else a
-    contiguous copy."""
-    es = t.element_size()
-    ok = t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all((s * es) % 16 == 0 for s in t.stride()[:-1])
-    return t if ok else t.contiguous()
+def ready16(t: torch.Tensor, tokens: Optional[int] = None) -> torch.Tensor:
+    """t itself when its last dimension is contiguous, its base and every
+    other stride are 16-byte aligned (the kernels' vector loads), and the
+    rows along the dimension `tokens`, if given, do not share memory
+    (distinct_rows); else a copy of its own (contiguous() would return a
+    contiguous t whatever its base)."""
+    *outer, last = t.stride()
+    if last == 1 and t.data_ptr() % 16 == 0 and (tokens is None or outer[tokens] >= t.shape[-1]):
+        es = t.element_size()
+        for s in outer:
+            if (s * es) % 16:
+                break
+        else:
+            return t
+    return t.clone(memory_format=torch.contiguous_format)
 
 
 # ------------------------------------------------------------ 512-token spectra

@@ -259,7 +259,7 @@ class OrthoCache_GQA_Attention:
         if nc is not None and (Hkv > nc.num_kv_heads or T > nc.max_tiles):
             raise IndexError(f"norm cache ({nc.num_kv_heads} heads x {nc.max_tiles} tiles) is smaller than the "
                              f"prefill ({Hkv} heads x {T} tiles)")
-        query, key, value = X.ready16(query), *(X.distinct_rows(X.ready16(t), 2) for t in (key, value))
+        query, key, value = X.ready16(query), X.ready16(key, 2), X.ready16(value, 2)
         # the norms ||(H64 K_t)[48:64]||_F of every complete tile, per q head
         # the lower median over positions of ||q||_2, the group's max, the
         # gate and its statistics, and the norm cache

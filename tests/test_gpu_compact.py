@@ -422,3 +422,30 @@ def test_block_spectra_of_keys_that_are_not_finite(dtype, d):
         np.testing.assert_allclose(np64(got[name]), ref[name], rtol=1e-5, atol=1e-6, err_msg=name)
     for b in (0, 2, 3):  # (block 1's energy is NaN, which its bounds take as none)
         np.testing.assert_allclose(np64(got["bounds"])[:, b], ref["bounds"][:, b], rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("shifted", ["q", "k", "v"])
+@pytest.mark.parametrize("Sq", [1, 20])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_dense_forward_of_a_contiguous_tensor_off_16_bytes(dtype, Sq, shifted):
+    """A contiguous tensor whose base is not 16-byte aligned is copied for the
+    query blocks' vector loads (torch's contiguous() returns it as it is, and
+    the library refused it)."""
+    from orthocache_gpu.adaptive_attention import attend_tiles
+    from orthocache_gpu.pipeline import orthocache_forward
+    H, S, d = 4, 256, 64
+    g = torch.Generator().manual_seed(19)
+    t = {}
+    for n, s in (("q", Sq), ("k", S), ("v", S)):
+        x = torch.randn((s * H * d + 1,), generator=g).to(TD[dtype]).to(DEV)
+        t[n] = (x[1:] if n == shifted else x[:-1]).view(s, H, d)
+    assert t[shifted].is_contiguous() and t[shifted].data_ptr() % 16
+    print(f"dense forward {dtype} Sq={Sq} shifted {shifted}", flush=True)
+    out, _ = orthocache_forward(t["q"], t["k"], t["v"], mode="dense")
+    masked = attend_tiles(t["q"], t["k"], t["v"], torch.ones(S // 64, dtype=torch.uint8, device=DEV), S)
+    q, k, v = (np64(t[n]) for n in "qkv")
+    logits = np.einsum("qhd,khd->hqk", q, k) / np.sqrt(d)
+    p = np.exp(logits - logits.max(axis=2, keepdims=True))
+    ref = np.einsum("hqk,khd->qhd", p / p.sum(axis=2, keepdims=True), v)
+    assert_out(out, ref, dtype, f"dense forward {dtype} Sq={Sq} shifted {shifted}")
+    assert_out(masked, ref, dtype, f"attend {dtype} Sq={Sq} shifted {shifted}")
