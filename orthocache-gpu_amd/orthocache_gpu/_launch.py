@@ -930,7 +930,7 @@ def prefill_gate(q: torch.Tensor, k: torch.Tensor, tau_norm: float, norm_scale: 
 
 def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, tile_mask: Optional[torch.Tensor] = None,
                       scale: Optional[float] = None, want_entropy: bool = False, split: bool = True,
-                      before_launch: Optional[Callable[[], None]] = None
+                      before_launch: Optional[Callable[[], None]] = None, prepared: bool = False
                       ) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
     """oc_prefill_attention: causal GQA attention of q (B, Hq, Sq, d) over k, v
     (B, Hkv, Skv, d) (last dimensions contiguous, other strides free),
@@ -940,10 +940,13 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, tile
     workgroups each when the call fits the device in one round (it then uses
     the stream's workspace).  before_launch() is called once nothing but the
     launch can fail any more: what it launches comes before the attention on
-    the stream, and may write tile_mask."""
-    device = check_prefill(q, k, v)
+    the stream, and may write tile_mask.  prepared: q, k and v have been
+    through check_prefill and ready16."""
+    if not prepared:
+        check_prefill(q, k, v)
+        q, k, v = ready16(q), ready16(k, 2), ready16(v, 2)
+    device = q.device
     B, Hq, Sq, d = q.shape
-    q, k, v = ready16(q), ready16(k, 2), ready16(v, 2)
     Hkv, Skv = k.shape[1], k.shape[2]
     out = torch.empty((B, Hq, Sq, d), dtype=q.dtype, device=device)
     ent = torch.empty((B, Hq, Sq), dtype=torch.float32, device=device) if want_entropy else None
