@@ -224,6 +224,52 @@ def test_prefill_gate_argument_checks():
     refused(N.OC_ERR_INVALID, b"norm cache", cache=256, cache_stride=1)
 
 
+def test_attend_argument_checks():
+    """oc_attend validates on the host; none of these calls launches."""
+    import ctypes
+    from orthocache_gpu import _native as N
+    L = N.lib()
+    assert L.oc_attend_params_bytes() == ctypes.sizeof(N.OcAttendParams)
+    good = dict(q=256, k=256, v=256, out=256, dtype=N.OC_BF16, out_dtype=N.OC_F32, num_heads=2, q_len=70, kv_len=500,
+                head_dim=64, q_stride_s=128, q_stride_h=64, k_stride_s=128, k_stride_h=64, v_stride_s=128,
+                v_stride_h=64, out_stride_s=128, out_stride_h=64, num_splits=4, workspace=256, workspace_bytes=1 << 30)
+
+    def refused(code, text, **change):
+        p = N.OcAttendParams()
+        for x, y in {**good, **change}.items():
+            setattr(p, x, y)
+        assert L.oc_attend(ctypes.byref(p), None) == code and text in L.oc_last_error(), change
+
+    assert L.oc_attend(None, None) == N.OC_ERR_INVALID
+    refused(N.OC_ERR_UNSUPPORTED, b"dtypes", dtype=N.OC_FP8_E4M3FN)
+    refused(N.OC_ERR_UNSUPPORTED, b"dtypes", out_dtype=N.OC_FP8_E4M3FN)
+    refused(N.OC_ERR_UNSUPPORTED, b"head_dim", head_dim=32)
+    refused(N.OC_ERR_INVALID, b"sizes", q_len=-1)
+    refused(N.OC_ERR_INVALID, b"sizes", num_splits=-1)
+    refused(N.OC_ERR_UNSUPPORTED, b"kv_len", kv_len=(1 << 20) + 1)
+    refused(N.OC_ERR_UNSUPPORTED, b"query blocks", num_heads=1 << 17, q_len=129 * 2)
+    for x in "qkv":
+        refused(N.OC_ERR_INVALID, b"NULL", **{x: None})
+        refused(N.OC_ERR_INVALID, b"aligned", **{x: 264})
+        refused(N.OC_ERR_INVALID, b"16 bytes", **{x + "_stride_s": 132})
+        refused(N.OC_ERR_INVALID, b"16 bytes", **{x + "_stride_h": 68})
+    refused(N.OC_ERR_INVALID, b"NULL", out=None)
+    refused(N.OC_ERR_INVALID, b"out not aligned", out=258)
+    for x in "kv":
+        refused(N.OC_ERR_UNSUPPORTED, b"stride too large", **{x + "_stride_s": 1 << 24})
+        refused(N.OC_ERR_INVALID, b"smaller than head_dim", **{x + "_stride_s": 0})
+    refused(N.OC_ERR_INVALID, b"one stride", out_stride_s=192)
+    refused(N.OC_ERR_WORKSPACE, b"workspace", workspace_bytes=1 << 16)
+    refused(N.OC_ERR_WORKSPACE, b"workspace", workspace=None)
+    # four shares of 70 x 2 rows: 64 KiB of another call's counters, alignment, acc, m and l
+    p = N.OcAttendParams()
+    for x, y in good.items():
+        setattr(p, x, y)
+    assert L.oc_attend_workspace_size(ctypes.byref(p)) == 65536 + 256 + 70 * 2 * 4 * 66 * 4
+    p.num_splits = 1
+    assert L.oc_attend_workspace_size(ctypes.byref(p)) == 0
+
+
 def test_spectra_argument_checks():
     import ctypes
     from orthocache_gpu import _native as N

@@ -449,3 +449,82 @@ def test_dense_forward_of_a_contiguous_tensor_off_16_bytes(dtype, Sq, shifted):
     ref = np.einsum("hqk,khd->qhd", p / p.sum(axis=2, keepdims=True), v)
     assert_out(out, ref, dtype, f"dense forward {dtype} Sq={Sq} shifted {shifted}")
     assert_out(masked, ref, dtype, f"attend {dtype} Sq={Sq} shifted {shifted}")
+
+
+def _softmax_rows(q, k, v, keep):
+    """softmax(q k^T / sqrt(d)) v in float64, keep (H, S): (Sq, H, d), zeros where a head keeps nothing."""
+    out = np.zeros(q.shape)
+    for h in range(q.shape[1]):
+        if keep[h].any():
+            x = q[:, h] @ k[keep[h], h].T / np.sqrt(q.shape[2])
+            p = np.exp(x - x.max(axis=1, keepdims=True))
+            out[:, h] = p / p.sum(axis=1, keepdims=True) @ v[keep[h], h]
+    return out
+
+
+@pytest.mark.parametrize("dtype,d", [("f32", 64), ("f32", 128), ("f16", 64), ("bf16", 128)])
+@pytest.mark.parametrize("splits", [1, 5])
+def test_attend_masks_per_head_in_another_dimension_order(dtype, d, splits):
+    """A mask row for each head (their counts of retained tiles differ, one
+    has none, one only the partial last tile) with K and V stored (H, S, d) and
+    q (H, Sq, d)."""
+    import ctypes
+    from orthocache_gpu import _launch as X
+    from orthocache_gpu import _native as N
+    H, Sq, S = 5, 37, 64 * 70 + 9
+    T = -(-S // 64)
+    g = torch.Generator().manual_seed(d + splits)
+    q, k, v = (torch.randn((H, n, d), generator=g).to(TD[dtype]).to(DEV).permute(1, 0, 2) for n in (Sq, S, S))
+    mask = (torch.rand((H, T + 3), generator=g) < torch.tensor([0.0, 0.9, 0.2, 0.02, 0.0])[:, None]).to(torch.uint8)
+    mask[3, T - 1] = 1
+    mask[4] = 0
+    mask[4, T - 1] = 1
+    mask_dev = mask.to(DEV)
+    out = torch.full((Sq, H, d), 9.0, dtype=torch.float32, device=DEV)
+    p = N.OcAttendParams()
+    for n, t in (("q", q), ("k", k), ("v", v), ("out", out)):
+        setattr(p, n, t.data_ptr())
+        setattr(p, n + "_stride_s", t.stride(0))
+        setattr(p, n + "_stride_h", t.stride(1))
+    p.dtype, p.out_dtype, p.num_heads, p.q_len, p.kv_len, p.head_dim = X.dtype_code(q.dtype, "q"), N.OC_F32, H, Sq, S, d
+    p.tile_mask, p.tile_mask_stride_h, p.scale, p.num_splits = mask_dev.data_ptr(), T + 3, d ** -0.5, splits
+    ws = torch.empty((N.lib().oc_attend_workspace_size(ctypes.byref(p)),), dtype=torch.uint8, device=DEV)
+    p.workspace, p.workspace_bytes = ws.data_ptr() if splits > 1 else None, ws.numel()
+    print(f"attend per head {dtype} d={d} splits={splits}", flush=True)
+    N.check("oc_attend", N.lib().oc_attend(ctypes.byref(p), ctypes.c_void_p(X.current_stream(out.device))))
+    keep = np.repeat(mask.numpy()[:, :T].astype(bool), 64, axis=1)[:, :S]
+    assert not keep[0].any() and keep[4].sum() == 9 and not out[:, 0].any()
+    assert_out(out, _softmax_rows(np64(q), np64(k), np64(v), keep), dtype, f"attend per head {dtype} d={d}")
+
+
+@pytest.mark.parametrize("dtype,d", [("f32", 64), ("f32", 128), ("f16", 64), ("bf16", 64), ("bf16", 128)])
+@pytest.mark.parametrize("S", [200, 4160])  # one share of a head's tiles, and several
+def test_attend_values_that_are_not_finite(dtype, d, S):
+    """Infinities and NaN stay with the head, query or column they are in: a
+    score of +inf or NaN makes a query NaN, one of -inf drops its token, a value
+    that is not finite reaches its own column only."""
+    from orthocache_gpu import _launch as X
+    H, Sq = 6, 20
+    g = torch.Generator().manual_seed(S + d)
+    q, k, v = (torch.randn((n, H, d), generator=g).to(TD[dtype]) for n in (Sq, S, S))
+    q[:, 1, 0] = q[:, 1, 0].abs() + 0.25
+    q[::2, 1, 0] *= -1
+    k[70, 1, 0] = -math.inf      # head 1: -inf against positive q, +inf against negative
+    k[70, 2, 0] = math.nan       # head 2: NaN for every query
+    q[7, 3, 0] = math.nan        # head 3: one query
+    v[70, 4, 5] = math.inf       # head 4: one column
+    v[71, 4, 6] = math.nan
+    q[:, 5, 0] = q[:, 5, 0].abs() + 0.25
+    k[:, 5, 0] = -math.inf       # head 5: every score -inf: nothing attended, as the decode kernels have it
+    print(f"attend not finite {dtype} d={d} S={S}", flush=True)
+    got = np64(X.attend(q.to(DEV), k.to(DEV), v.to(DEV), torch.float32))
+    with np.errstate(invalid="ignore"):
+        ref = _softmax_rows(np64(q), np64(k), np64(v), np.ones((H, S), dtype=bool))
+    assert np.isnan(ref[::2, 1]).all() and np.isfinite(ref[1::2, 1]).all() and np.isnan(ref[:, 2]).all()
+    assert not np.isfinite(got[:, 4, 5:7]).any() and not np.isfinite(ref[:, 4, 5:7]).any()
+    assert np.isnan(ref[:, 5]).all() and not got[:, 5].any()
+    for x in (got, ref):
+        x[:, 4, 5:7] = 0.0
+        x[:, 5] = 0.0
+    assert np.array_equal(np.isnan(got), np.isnan(ref)) and not np.isinf(got).any()
+    assert_out(np.nan_to_num(got), np.nan_to_num(ref), dtype, f"attend not finite {dtype} d={d} S={S}")
