@@ -923,8 +923,14 @@ def prefill_gate(q: torch.Tensor, k: torch.Tensor, tau_norm: float, norm_scale: 
     p.q_norms, p.k_norms, p.mask, p.gate_stats = qn.data_ptr(), kn.data_ptr(), mask.data_ptr(), _ptr(stats_out)
     if cache is not None:
         p.cache, p.cache_stride, p.valid_tiles = cache.data_ptr(), cache.stride(0), _ptr(valid_tiles)
-    with torch.cuda.device(device):
-        N.check("oc_prefill_gate", N.lib().oc_prefill_gate(ctypes.byref(p), ctypes.c_void_p(current_stream(device))))
+    stream = ctypes.c_void_p(current_stream(device))
+    if device.index == torch.cuda.current_device():
+        rc = N.lib().oc_prefill_gate(ctypes.byref(p), stream)
+    else:
+        with torch.cuda.device(device):
+            rc = N.lib().oc_prefill_gate(ctypes.byref(p), stream)
+    if rc:
+        N.check("oc_prefill_gate", rc)
     return mask, kn
 
 

@@ -279,6 +279,7 @@ class OrthoCache_GQA_Attention:
 
         want_entropy = self.governor is not None and hasattr(self.governor, 'set_entropy')
         out, ent = X.prefill_attention(query, key, value, tile_mask=evict, want_entropy=want_entropy,
+                                       split=False,  # a masked call does not split: no workspace to ask for
                                        before_launch=gate, prepared=True)
         if nc is not None:
             if not in_kernel:
