@@ -947,8 +947,7 @@ __device__ __forceinline__ const char* page_row(const char* pool, int64_t blk_st
 // four lanes of a token cover 64 bytes without a gap, as in 16 bits.  (With the
 // D/4 consecutive bytes kg*D/4 .. per lane, a load touched 16 bytes of every
 // D/4: 32 rows x 32768 tokens of 256, G = 8, half retained, 116.5 -> 95.0 us
-// single pass and 81.0 -> 66.1 cached; of 128, 131072 tokens, 153.7 -> 150.6
-// single pass on one box.)
+// single pass and 81.0 -> 66.1 cached; at 128 within the spread of one side.)
 template <int DT, int D, bool PAGED>
 __device__ __forceinline__ void load_k_mfma(const DecodeArgs& a, const RowInfo& ri, int row, int t, int lane,
                                             uint32_t (&kb)[4][D / 32][4], const TilePages& pg) {

@@ -192,9 +192,10 @@ __device__ __forceinline__ void pf_load_q(const PrefillArgs& a, const char* qh, 
 }
 
 // The workgroup's shared K/V tiles: K and V of one 64-token tile, row-major
-// [token][D], in STAGES LDS stages.  The 256 threads stage the next tile
-// through registers: each loads its 16-byte chunks while the waves compute
-// the current tile, and stores them once that compute is done.  K's chunks
+// [token][D], in STAGES LDS stages.  The 512 threads stage the next tile, in
+// 16-byte chunks, while the waves compute the current one: straight into the
+// other stage where there are two, else (float32 at head_dim 128) through
+// registers, stored once that compute is done.  K's chunks
 // are XOR-swizzled per row (chunk c of row r sits at c ^ swz(r)) so that the
 // 16 rows one B-operand read touches fall in distinct LDS banks.
 template <int DT, int D>
@@ -232,7 +233,7 @@ __device__ __forceinline__ const char* pf_uniform(const char* p) {
   return reinterpret_cast<const char*>(((uint64_t)hi << 32) | lo);
 }
 
-// global -> registers: chunk g = tid + 256 j of the tile is row g / LPT,
+// global -> registers: chunk g = tid + 512 j of the tile is row g / LPT,
 // chunk g % LPT; rows at or past kv_len read as zero (buffer range check)
 template <int DT, int D>
 __device__ __forceinline__ void pf_fetch(const PrefillArgs& a, const char* kh, const char* vh, int t, int tid,
@@ -369,8 +370,9 @@ __device__ __forceinline__ void pf_logits(const PfQ<DT, D>& q, const char* sk, i
 // the lane's own eight probabilities c[2j][b], c[2j + 1][b].  HILO sends a
 // 16-bit high part plus the 16-bit rounding of the remainder (two
 // instructions); without it they are rounded once, which the causal kernel
-// does for float16 (relative error at most 2^-12): in bfloat16 one rounding
-// (2^-9) moves short causal rows past the output tolerance.
+// does for float16 (relative error at most 2^-11; below 2^-14, where float16 is
+// subnormal, an absolute 2^-25): in bfloat16 one rounding (2^-8) moves short
+// causal rows past the output tolerance.
 // float32: 16x16x4 steps over (tb, i), A = V[16tb + 4r + i][16nc + x], B =
 // c[tb][i], exact.
 template <int DT, int D, bool HILO = DT == OC_BF16>

@@ -781,7 +781,8 @@ def row_norms(x: torch.Tensor, low_band: int = 0) -> torch.Tensor:
 
 def kth_smallest(x: torch.Tensor, k: int) -> torch.Tensor:
     """oc_kth_smallest: the k-th smallest (0-based) of each row of a float32
-    (rows, n) tensor of non-negative values."""
+    (rows, n) tensor of non-negative values.  (The C entry point's binding; the
+    hook's prefill selects inside oc_prefill_gate.)"""
     device = require_gpu(x)
     if x.dtype != torch.float32 or x.dim() != 2 or x.stride(1) != 1:
         x = x.to(torch.float32).contiguous().reshape(x.shape[0], -1)
@@ -795,7 +796,9 @@ def kth_smallest(x: torch.Tensor, k: int) -> torch.Tensor:
 
 def group_gate(q_norms: torch.Tensor, k_norms: torch.Tensor, num_kv_heads: int, G: int, num_tiles: int,
                mask_cols: int, tau_norm: float, reduce: int, keep_polarity: bool = False, want_stats: bool = False):
-    """oc_group_gate.  q_norms: float32 (batch, num_kv_heads * G); k_norms:
+    """oc_group_gate (the C entry point's binding; the hook gates inside
+    oc_prefill_gate and oc_hook_decode).  q_norms: float32 (batch, num_kv_heads
+    * G); k_norms:
     float32 (batch or 1, num_kv_heads, >= num_tiles) (a batch of 1 is shared
     by every batch entry).  Returns (mask uint8 (batch, num_kv_heads,
     mask_cols), group norms float32 (batch, num_kv_heads)), plus with
@@ -826,12 +829,20 @@ def attend_takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
     """Whether q (Sq, H, d) over k, v (S, H, d) goes to oc_attend rather than
     to the decode kernels: one float type, head_dim 64 or 128, at most 1M
     tokens, and more than one query in 16 bits, more than eight in float32.
-    Half the tiles retained, 32 heads of 128, decode against oc_attend in us:
-    bfloat16 over 32768 tokens 54 / 60 for one query, 63 / 60 for two, 96 / 61
-    for nine and 313 / 75 for 70; float32 over 16384 tokens 81 / 102 for eight
-    and 123 / 102 for nine (the decode holds a float32 tile in registers, the
-    query block stages it through LDS).  Eight is what the decode kernels take
-    in one pass over a head's K and V."""
+    Half the tiles retained, 32 heads of 128, the kernels of the decode against
+    oc_attend's in us: bfloat16 over 32768 tokens 54 / 60 for one query, 63 / 60
+    for two, 96 / 61 for nine and 313 / 75 for 70; float32 over 16384 tokens 81 /
+    102 for eight and 123 / 102 for nine (the decode holds a float32 tile in
+    registers, the query block stages it through LDS).  Eight is what the decode
+    kernels take in one pass over a head's K and V.
+
+    Over 1, 8, 32 and 64 heads of 64 and 128, 512 to 131072 tokens, masked and
+    dense, two to eight 16-bit queries: calls 29-49 us by the decode, 18-24 by
+    oc_attend where the host bounds them (the decode also copies q and the
+    output), and captured, without the host, 0.5 to 0.97 of the decode's time;
+    one head of 64 alone is the slower there by up to 1.3 us (4096 tokens, two
+    queries, dense: 11.2 / 12.4).  From nine float32 queries on a call is never
+    slower but for one head of 128, dense, waited for (49 / 51 at 4096 tokens)."""
     if q.shape[0] <= (8 if q.dtype == torch.float32 else 1):
         return False
     # what oc_attend refuses (rows 2^22 elements or more apart, over 2^17 query

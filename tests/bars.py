@@ -13,7 +13,7 @@ that type.  assert_out therefore checks, element by element,
                                     of the reference (golden vectors)
 
 and records the achieved max-abs error beside the plain bar.  h is at
-most 2^-9 |ref| in bfloat16 and 2^-12 |ref| in float16, so for outputs
+most 2^-8 |ref| in bfloat16 and 2^-11 |ref| in float16, so for outputs
 below 0.5 in magnitude (nearly all decode outputs: averages of many value
 rows) the check is the plain bar; the terminal summary lists the worst
 error per bar and every check whose plain max-abs error exceeded its bar.
