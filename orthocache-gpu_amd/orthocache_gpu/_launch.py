@@ -837,11 +837,11 @@ def attend_takes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
     kernels take in one pass over a head's K and V.
 
     Over 1, 8, 32 and 64 heads of 64 and 128, 512 to 131072 tokens, masked and
-    dense, two to eight 16-bit queries: calls 29-49 us by the decode, 18-24 by
+    dense, two to eight 16-bit queries: calls 29-39 us by the decode, 18-24 by
     oc_attend where the host bounds them (the decode also copies q and the
-    output), and captured, without the host, 0.5 to 0.97 of the decode's time;
-    one head of 64 alone is the slower there by up to 1.3 us (4096 tokens, two
-    queries, dense: 11.2 / 12.4).  From nine float32 queries on a call is never
+    output), and captured, without the host, 0.5 to 0.96 of the decode's time
+    from eight heads on; one head of 128 is level there and one of 64 the
+    slower by up to 1.3 us (4096 tokens, two queries, dense: 11.2 / 12.4).  From nine float32 queries on a call is never
     slower but for one head of 128, dense, waited for (49 / 51 at 4096 tokens)."""
     if q.shape[0] <= (8 if q.dtype == torch.float32 else 1):
         return False
